@@ -487,6 +487,9 @@ struct gsdh_model {
         uint4* xa = nullptr;                      // hi/lo MFMA fragments
         float* xs = nullptr;                      // per-token descales
         float* tmp = nullptr;                     // rank-k values [kMaxSeg][chunk][kMaxRank]
+        // second buffers of the 32 x 32 tile path: a projection's result is
+        // taken in by the pass that prepares the next input
+        float *xn1 = nullptr, *xs1 = nullptr, *tmp1 = nullptr;
         float* part = nullptr;                    // split partials
         size_t part_bytes = 0;
         int chunk = 0;
@@ -725,6 +728,23 @@ int issue_head(gsdh_model* m, bool greedy) {
     return 0;
 }
 
+// The step's attention of layer l: any position (split, merged) or, with
+// short_chunk, positions below it (one block per KV head).
+AttnArgs layer_attention(gsdh_model* m, int l, int short_chunk) {
+    const auto& c = m->c;
+    AttnArgs a{};
+    a.q = m->q; a.k_cache = m->kc; a.v_cache = m->vc; a.out = m->attn; a.pos_dev = &m->st->pos;
+    a.layer = l; a.n_heads = c.n_heads; a.n_kv = c.n_kv_heads; a.hd = c.head_dim; a.max_seq = c.max_seq_len;
+    a.sm_scale = 1.0f / (float)std::sqrt((double)c.head_dim);
+    a.chunk = m->chunk; a.max_splits = m->max_splits; a.ws = m->ws; a.counters = m->counters;
+    a.err = &m->st->err;
+    if (short_chunk) {
+        a.chunk = short_chunk;
+        a.max_splits = 1;
+    }
+    return a;
+}
+
 // The per-token launch sequence (run_gpu_native_chat.py:892-969, fused).
 // short_chunk: 0 for the graph of any position, else the single attention
 // chunk (64, 128 or 256) of the graph for positions below it
@@ -751,17 +771,7 @@ int issue_token(gsdh_model* m, bool with_head, int short_chunk) {
             r.interleaved = 0;
             HIPCHK(launch_rope_kv(m->q, m->k, m->v, r, nullptr, m->stream));
         }
-        AttnArgs a{};
-        a.q = m->q; a.k_cache = m->kc; a.v_cache = m->vc; a.out = m->attn; a.pos_dev = &m->st->pos;
-        a.layer = l; a.n_heads = c.n_heads; a.n_kv = c.n_kv_heads; a.hd = c.head_dim; a.max_seq = c.max_seq_len;
-        a.sm_scale = 1.0f / (float)std::sqrt((double)c.head_dim);
-        a.chunk = m->chunk; a.max_splits = m->max_splits; a.ws = m->ws; a.counters = m->counters;
-        a.err = &m->st->err;
-        if (short_chunk) {   // positions < short_chunk: one block per KV head
-            a.chunk = short_chunk;
-            a.max_splits = 1;
-        }
-        HIPCHK(launch_attention(a, m->stream));
+        HIPCHK(launch_attention(layer_attention(m, l, short_chunk), m->stream));
         rc = issue_linear(m, l, 2 | 4 | 8);
         if (rc) return rc;
     }
@@ -792,6 +802,55 @@ size_t split_part_bytes(int M, int rows, int cols) {   // the prefill's (high + 
     return plan.nsplit > 1 ? (size_t)plan.nsplit * ((M + 15) / 16 * 16) * rows * 4 : 0;
 }
 
+MmSeg mm_seg(const HexDev& t, float* Y) {
+    MmSeg w{};
+    w.codes_t = t.codes_t; w.scales_t = t.scales_t; w.row_ptr = t.nk ? t.row_ptr : nullptr; w.kcols = t.kcols;
+    w.kdel = t.kdel; w.U = t.U; w.Y = Y; w.rows = t.rows; w.k = t.k;
+    return w;
+}
+
+// Whether the model's prompts run on the 32 x 32 tile projections
+// (issue_prompt32): in every layer the tensors that share an input of one
+// covered codebook, ranks of at most 2 (layer_prep_kernel's), rows within
+// its LDS.  Other models keep issue_prefill.
+bool prompt_mm32(gsdh_model* m) {
+    const auto& c = m->c;
+    if (c.hidden > kLayerPrepMaxCols || c.ffn > kLayerPrepMaxCols || c.n_heads * c.head_dim > kLayerPrepMaxCols) return false;
+    for (int l = 0; l < c.n_layers; l++) {
+        for (int s = 0; s < 7; s++) {
+            const HexDev& t = m->slot(l, s);
+            if (t.k > 2 || !hexmm32_codebook(3 * t.radius * t.radius + 3 * t.radius + 1)) return false;
+        }
+        const int r = m->slot(l, GSDH_Q).radius;
+        if (m->slot(l, GSDH_K).radius != r || m->slot(l, GSDH_V).radius != r ||
+            m->slot(l, GSDH_GATE).radius != m->slot(l, GSDH_UP).radius)
+            return false;
+    }
+    return true;
+}
+
+// Partial sums of the 32 x 32 tile projections of an M-token chunk (M and
+// the up to 15 fewer tokens of its last group tile alike)
+size_t prompt_part_bytes(gsdh_model* m, int M) {
+    if (!prompt_mm32(m)) return 0;
+    const auto& c = m->c;
+    const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim;
+    const int sets[5][4] = {{qd, kvd, kvd, c.hidden}, {kvd, kvd, 0, c.hidden}, {c.hidden, 0, 0, qd}, {c.ffn, c.ffn, 0, c.hidden},
+                            {c.hidden, 0, 0, c.ffn}};
+    size_t n = 0;
+    for (const auto& st : sets) {
+        MmArgs a{};
+        a.M = M;
+        int tiles = 0, grid = 0;
+        for (a.nseg = 0; a.nseg < kMaxSeg && st[a.nseg]; a.nseg++) {
+            a.seg[a.nseg].rows = st[a.nseg];
+            tiles += (st[a.nseg] + 15) / 16;
+        }
+        n = std::max(n, hexmm32_layout(a, hexmm32_tile_hl(M, tiles, st[3]), &grid) * 4);
+    }
+    return n;
+}
+
 // The batched workspaces, sized for every tensor shape of the model and every
 // batch size up to the limits, so no later call allocates.
 int setup_batched(gsdh_model* m) {
@@ -805,6 +864,7 @@ int setup_batched(gsdh_model* m) {
             if (M <= kPrefillChunk) part = std::max(part, split_part_bytes(M, sh[0], sh[1]));
         }
         mm = std::max(mm, matmul_ws_need(M, c.vocab, c.hidden));
+        if (M <= kPrefillChunk && M % 16 == 0) part = std::max(part, prompt_part_bytes(m, M));
     }
     auto& P = m->pf;
     const int Mc = kPrefillChunk, Mp = (Mc + 15) / 16 * 16;
@@ -828,6 +888,11 @@ int setup_batched(gsdh_model* m) {
     A((void**)&P.xs, (size_t)Mp * 4);
     A((void**)&P.tmp, (size_t)kMaxSeg * Mc * kMaxRank * 4);
     A((void**)&P.part, part);
+    if (prompt_mm32(m)) {
+        A((void**)&P.xn1, (size_t)Mp * maxc * 4);
+        A((void**)&P.xs1, (size_t)Mp * 4);
+        A((void**)&P.tmp1, (size_t)kMaxSeg * Mc * kMaxRank * 4);
+    }
     return rc;
 }
 
@@ -926,6 +991,92 @@ int issue_prefill(gsdh_model* m, int M, int p0) {
     return 0;
 }
 
+// Prompt tokens P.tok[0..M) at positions p0.. on the 32 x 32 tile
+// projections, what issue_prefill computes: q, k and v in one launch, gate
+// and up in one, and each projection's column splits, descale, kink, rank-k,
+// residual and SwiGLU terms taken in by the pass that prepares the next
+// input.  9 launches per layer instead of 19.  x is then the last token's.
+int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
+    const auto& c = m->c;
+    auto& P = m->pf;
+    const int qd = c.n_heads * c.head_dim;
+    int rc = 0, at = 0;   // `at`: which of the two sets of input buffers the coming projections read
+    float* const xn[2] = {P.xn, P.xn1};
+    float* const xs[2] = {P.xs, P.xs1};
+    float* const tm[2] = {P.tmp, P.tmp1};
+    MmArgs a{};           // the last projection
+    // the input `in` of tensors ts[0..n) prepared, then their projection
+    // into Y[i] (added to it with accumulate) or, split, as partial sums
+    auto project = [&](LayerPrepIn kind, float* X, const float* norm_w, int cols, const int* slots, int n, int l,
+                       float* const* Y, bool accumulate) -> int {
+        at ^= 1;
+        LayerPrep p{};
+        p.X = X; p.embed = m->embed; p.tokens = P.tok; p.in = a.in; p.part = P.part;
+        for (int s = 0; s < 2 && s < a.nseg; s++) p.last[s] = a.seg[s];
+        p.norm_w = norm_w; p.eps = c.rms_eps; p.M = M; p.cols = cols; p.xa = P.xa; p.xs = xs[at];
+        MmArgs b{};
+        b.nseg = n; b.M = M; b.hl = 1; b.accumulate = accumulate; b.xa = P.xa; b.part = P.part;
+        b.in.xs = xs[at]; b.in.cols = cols;
+        int tiles = 0;
+        for (int s = 0; s < n; s++) {
+            const HexDev& t = m->slot(l, slots[s]);
+            b.seg[s] = mm_seg(t, Y[s]);
+            b.n_pts = 3 * t.radius * t.radius + 3 * t.radius + 1;
+            b.fields = m->fields[t.radius];
+            tiles += (t.rows + 15) / 16;
+            if (t.nk) p.xn = xn[at];
+            if (t.k > 0) {
+                p.Vt[s] = t.Vt; p.S[s] = t.Sv; p.k[s] = t.k;
+                p.tmp[s] = tm[at] + (size_t)s * P.chunk * kMaxRank;
+                b.seg[s].tmp_k = p.tmp[s];
+            }
+        }
+        b.in.Xf = p.xn;
+        int grid = 0;
+        if (hexmm32_layout(b, hexmm32_tile_hl(M, tiles, cols), &grid) * 4 > P.part_bytes)
+            return fail(-1, "prefill: split partials of %d tokens exceed the workspace", M);
+        HIPCHK(launch_layer_prep(p, kind, m->stream));
+        HIPCHK(launch_hexmm32(b, grid, m->stream));
+        a = b;
+        return 0;
+    };
+    static const int kQkv[3] = {GSDH_Q, GSDH_K, GSDH_V}, kO[1] = {GSDH_O}, kGu[2] = {GSDH_GATE, GSDH_UP}, kDown[1] = {GSDH_DOWN};
+    float* const qkv[3] = {P.Q, P.K, P.V};
+    float* const xo[1] = {P.X};
+    float* const gu[2] = {P.G, P.U};
+    for (int l = 0; l < c.n_layers; l++) {
+        // (a projection into X that was not split is in X already)
+        LayerPrepIn in = l == 0 ? kPrepEmbed : (a.seg[0].nsplit > 1 ? kPrepResidual : kPrepRow);
+        if ((rc = project(in, P.X, m->norm(l, 0), c.hidden, kQkv, 3, l, qkv, false))) return rc;
+        QkvFinish f{};
+        for (int s = 0; s < a.nseg; s++) f.last[s] = a.seg[s];
+        f.nseg = a.nseg; f.M = M; f.in = a.in; f.part = P.part; f.q = P.Q;
+        f.r.cs = m->cs; f.r.pos = p0; f.r.k_cache = m->kc; f.r.v_cache = m->vc; f.r.layer = l; f.r.n_heads = c.n_heads;
+        f.r.n_kv = c.n_kv_heads; f.r.hd = c.head_dim; f.r.max_seq = c.max_seq_len; f.r.interleaved = c.rope_interleaved;
+        // (an unsplit projection left q in P.Q: rotated in place)
+        HIPCHK(launch_qkv_finish(f, m->stream));
+        PrefillAttn pa{};
+        pa.q = P.Q; pa.k_cache = m->kc; pa.v_cache = m->vc; pa.out = P.A; pa.layer = l; pa.p0 = p0; pa.M = M;
+        pa.n_heads = c.n_heads; pa.n_kv = c.n_kv_heads; pa.hd = c.head_dim; pa.max_seq = c.max_seq_len;
+        pa.sm_scale = 1.0f / (float)std::sqrt((double)c.head_dim);
+        HIPCHK(launch_prefill_attention(pa, m->stream));
+        if ((rc = project(kPrepRow, P.A, nullptr, qd, kO, 1, l, xo, true))) return rc;
+        in = a.seg[0].nsplit > 1 ? kPrepResidual : kPrepRow;
+        if ((rc = project(in, P.X, m->norm(l, 1), c.hidden, kGu, 2, l, gu, false))) return rc;
+        if ((rc = project(kPrepSwiGLU, nullptr, nullptr, c.ffn, kDown, 1, l, xo, true))) return rc;
+    }
+    if (!last) return 0;
+    if (a.seg[0].nsplit == 1) {
+        HIPCHK(hipMemcpyAsync(m->x, P.X + (size_t)(M - 1) * c.hidden, (size_t)c.hidden * 4, hipMemcpyDeviceToDevice, m->stream));
+        return 0;
+    }
+    LayerPrep p{};   // the last layer's down, and the last token's row of it
+    p.X = P.X; p.in = a.in; p.part = P.part; p.last[0] = a.seg[0]; p.M = M; p.cols = c.hidden; p.xa = P.xa;
+    p.xs = xs[at ^ 1]; p.xlast = m->x;
+    HIPCHK(launch_layer_prep(p, kPrepResidual, m->stream));
+    return 0;
+}
+
 // Prompt prompt[0..n) at positions start.. in batches of the prefill chunk;
 // with `head`, the last token's logits and the greedy step (the step state
 // then holds the first generated token at position start + n, gen_count 1).
@@ -935,18 +1086,21 @@ int issue_prefill(gsdh_model* m, int M, int p0) {
 // chunk's attention reaches the caller.
 int run_prefill(gsdh_model* m, const int* prompt, int n, int start, bool head, int* tok_stage) {
     auto& P = m->pf;
-    HIPCHK(launch_set_step(m->st, prompt[0], start, 1, m->stream));
+    HIPCHK(launch_set_step(m->st, prompt[n - 1], start + n - 1, 1, m->stream));
     for (int b0 = 0; b0 < n; b0 += P.chunk) {
         const int M = std::min(P.chunk, n - b0);
         int* ts = tok_stage + b0;
         for (int i = 0; i < M; i++) ts[i] = prompt[b0 + i];
         HIPCHK(hipMemcpyAsync(P.tok, ts, (size_t)M * 4, hipMemcpyHostToDevice, m->stream));
-        int rc = issue_prefill(m, M, start + b0);
+        int rc = P.xs1 ? issue_prompt32(m, M, start + b0, b0 + M == n) : issue_prefill(m, M, start + b0);
         if (rc) return rc;
     }
-    HIPCHK(launch_set_step(m->st, prompt[n - 1], start + n - 1, 0, m->stream));
-    if (head) return issue_head(m, true);
-    return 0;
+    if (!head) return 0;
+    // the head takes its publication words (ranks above 2) from the first
+    // on, cleared: each prompt took the next ones until none were left
+    m->pub_next = 0;
+    if (m->slot(0, GSDH_LM_HEAD).k > 2) HIPCHK(launch_fill_u32((unsigned*)m->pub, 0u, 2 * (size_t)kLeadMax, m->stream));
+    return issue_head(m, true);
 }
 
 int capture(gsdh_model* m, bool with_head, int short_chunk, hipGraphExec_t* out) {

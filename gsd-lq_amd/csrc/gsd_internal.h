@@ -266,6 +266,96 @@ hipError_t launch_hexmm_prepared(const MatmulArgs& a, hipStream_t stream);
 // X[m][:] = fp16 embedding row of tokens[m] (fp32 [M][hidden])
 hipError_t launch_embed_rows(const uint16_t* embed, const int* tokens, int M, float* X, int hidden,
                              hipStream_t stream);
+// Column splits of nc chunks, ceil(nc / s) chunks each, none of them empty
+// (an empty split's partial sums would be read and never written)
+inline int whole_splits(int nc, int s) {
+    const int per = (nc + s - 1) / s;
+    return (nc + per - 1) / per;
+}
+
+// Batched projection of up to kMaxSeg tensors of one codebook that read the
+// same operands, on 32 x 32 matrix-core tiles, in one launch (gsd_prefill.hip).
+// A tensor's columns may be split: its partial sums then lie at part + p0
+// ([nsplit][ceil(M/16)*16][rows]) and whoever reads the result adds them, in
+// split order, and the descale, kink and rank-k terms (mm_finish).
+struct MmSeg {
+    const uint4* codes_t;
+    const uint32_t* scales_t;
+    const uint32_t* row_ptr;   // null: no kinks
+    const uint16_t* kcols;
+    const float* kdel;
+    const uint16_t* U;         // k > 0
+    const float* tmp_k;        // k > 0: [M][k]
+    float* Y;                  // [M][rows]; nsplit == 1 writes it
+    size_t p0;
+    int rows, k, nsplit;
+    int b0;                    // the tensor's first block (a multiple of 8)
+};
+// What a projection's result still needs of its input: the per-token descale
+// and, for the kink terms, the input itself (fp32, or bf16)
+struct MmIn {
+    const float* xs;
+    const float* Xf;
+    const uint16_t* X;
+    int cols;
+};
+struct MmArgs {
+    MmSeg seg[kMaxSeg];
+    int nseg, n_pts, M, hl, accumulate;
+    int r2, t2;                // 32-row tiles per wave, 32-token tiles per block
+    const uint32_t* fields;
+    const uint4* xa;
+    MmIn in;
+    float* part;
+};
+struct MmTile {
+    int r2, t2, nsplit;
+};
+bool hexmm32_codebook(int n_pts);   // whether launch_hexmm32 covers the codebook
+MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols);
+size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid);
+hipError_t launch_hexmm32(const MmArgs& a, int grid, hipStream_t stream);
+// every split tensor's partial sums -> its Y (rows a multiple of 4)
+hipError_t launch_mm_reduce(const MmArgs& a, hipStream_t stream);
+
+// Operands of the next projections of a prompt's tokens (layer_prep_kernel):
+// from the rows X, from X plus the last projection (written back to X), from
+// silu(gate) * up of the last two, or from the tokens' embedding rows
+// (written to X).  Ranks of at most 2; every pointer 16-byte aligned.
+enum LayerPrepIn { kPrepRow, kPrepResidual, kPrepSwiGLU, kPrepEmbed };
+constexpr int kLayerPrepMaxCols = 32768;
+struct LayerPrep {
+    float* X;                  // [M][cols]
+    const uint16_t* embed;
+    const int* tokens;
+    MmSeg last[2];             // the projections taken in, with their input
+    MmIn in;
+    const float* part;
+    const float* norm_w;       // or null
+    float eps;
+    int M, cols;
+    uint4* xa;
+    float* xs;                 // (not the buffer in.xs points to)
+    float* xn;                 // [M][cols] for the kink terms, or null (not in.Xf)
+    float* xlast;              // the last token's row of X, too, or null
+    const uint16_t* Vt[kMaxSeg];
+    const float* S[kMaxSeg];
+    int k[kMaxSeg];
+    float* tmp[kMaxSeg];       // (not what last[].tmp_k points to)
+};
+hipError_t launch_layer_prep(const LayerPrep& p, LayerPrepIn in, hipStream_t stream);
+// RoPE and fp16 K/V append of M prompt tokens at r.pos .. from their q, k and
+// v projections (nseg 3; q: [M][n_heads * hd]) or k and v alone (nseg 2)
+struct QkvFinish {
+    MmSeg last[kMaxSeg];
+    int nseg, M;
+    MmIn in;
+    const float* part;
+    float* q;
+    RopeKV r;
+};
+hipError_t launch_qkv_finish(const QkvFinish& p, hipStream_t stream);
+
 // Tiling of a batched projection: token groups per block (tg: 1, 2, 4, 8),
 // row blocks per wave (rbw) and column splits (nsplit), chosen so the grid
 // fills the chip with the fewest re-decodes of the weights.

@@ -3846,7 +3846,7 @@ MatmulPlan hexmm_plan(int M, int rows, int cols, bool hl) {
         const int t8 = ((nrb + 15) / 16) * ((ng + 7) / 8);
         if (4 * t8 < 3 * ncu) {
             const int s = std::min((ncu + t8 - 1) / t8, std::max(1, nc / 4));
-            return MatmulPlan{8, 2, s};
+            return MatmulPlan{8, 2, whole_splits(nc, s)};
         }
     }
     for (int tg = 8; tg >= 1; tg >>= 1) {
@@ -3859,7 +3859,7 @@ MatmulPlan hexmm_plan(int M, int rows, int cols, bool hl) {
     int s = (2 * ncu + tiles - 1) / tiles;
     s = std::min(s, std::max(1, nc / 4));
     const long long cap = ((long long)rows * cols) / (4LL * (ng * 16) * rows);
-    p.nsplit = (int)std::max<long long>(1, std::min<long long>(s, cap));
+    p.nsplit = whole_splits(nc, (int)std::max<long long>(1, std::min<long long>(s, cap)));
     return p;
 }
 

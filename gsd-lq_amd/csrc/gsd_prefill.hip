@@ -1,0 +1,665 @@
+// gsd_prefill.hip -- the batched projection on 32 x 32 matrix-core tiles and
+// the kernels between the projections of a prompt's layers (no reference
+// kernel: the reference prefills token by token, run_gpu_native_chat.py:
+// 1128-1130).
+#include <algorithm>
+#include <type_traits>
+
+#include "gsd_device.h"
+#include "gsd_internal.h"
+
+// LDS addresses are formed as integers (an entry's address in one and-or, the
+// base in the instruction's offset), and the LDS loads of lds_dma16 take theirs in m0
+#pragma clang diagnostic ignored "-Wint-to-pointer-cast"
+#pragma clang diagnostic ignored "-Winline-asm"
+
+namespace gsd {
+namespace {
+
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) const uint32_t lds_u32;
+typedef __attribute__((address_space(3))) const u32x4v lds_u4;
+
+// LDS byte address code * 128 + off (off < 128) of code j, a constant, of a
+// lane's (aligned) word: 32 copies of an entry, one per lane of a half wave
+template <bool B7>
+__device__ __forceinline__ uint32_t code_addr32(const uint32_t (&w)[4], int j, uint32_t off) {
+    if (B7) {
+        const int s = 7 * j - 7, d = s >> 5;
+        const uint32_t x = j == 0 ? w[0] << 7 : (d == 3 ? w[3] >> (s & 31) : __builtin_amdgcn_alignbit(w[d + 1], w[d], s & 31));
+        return (x & 0x3F80u) | off;
+    }
+    const int b = j & 3;
+    const uint32_t x = b == 0 ? w[j >> 2] << 7 : w[j >> 2] >> (8 * b - 7);
+    return (x & 0x7F80u) | off;
+}
+
+// 64 lanes x 16 bytes from global memory into LDS at byte lds + 16 * lane,
+// past the registers (no output register, so nothing is allocated to the
+// load in flight; the caller waits on vmcnt before any wave reads the bytes)
+__device__ __forceinline__ void lds_dma16(const void* p, uint32_t lds) {
+    __asm__ volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
+}
+
+// y of one (token, row): the descaled sum s, kinks, rank-k
+__device__ __forceinline__ float mm_finish(const MmSeg& w, const MmIn& in, int m, int row, float s) {
+    float y = s * in.xs[m];
+    if (w.row_ptr) {
+        const uint32_t e = w.row_ptr[row + 1];
+        for (uint32_t j = w.row_ptr[row]; j < e; j++) {
+            const size_t at = (size_t)m * in.cols + w.kcols[j];
+            y += w.kdel[j] * (in.Xf ? in.Xf[at] : __uint_as_float((uint32_t)in.X[at] << 16));
+        }
+    }
+    for (int j = 0; j < w.k; j++) y += h2f(w.U[(size_t)row * w.k + j]) * w.tmp_k[(size_t)m * w.k + j];
+    return y;
+}
+
+// ------------------------------------------------------------------------
+// Batched projection, 32 x 32 x 16 matrix-core tiles.  Lattice form, packed
+// tiles and operand fragments as hexmm_kernel: A = the tokens' (u, v) as
+// fp16 (HL: high and low parts, two products per step), B = the rows'
+// integer fields (r0, r1), exact, from the codebook in LDS; a 64-column
+// block's sum is scaled by its fp16 scale into the fp32 accumulator.
+//
+// A block is 4 waves, each 32 R2 rows, over the same 32 T2 tokens, two
+// blocks per CU.  Bound: the matrix cores and, between them, the latency of
+// the operands.  What the layout is for:
+//  * 32 x 32 tiles: one wave per SIMD issues 1.9 PFLOP/s of them and 1.1 of
+//    16 x 16 tiles (fp16, measured alone), two waves 2.06 against 1.72;
+//  * a lane's half of a 32-row tile comes from lanes (l & 15) + 32 (l >> 5)
+//    and + 16 of the two 16-row tiles in memory, so neither the weights nor
+//    the operands change their layout: step s = 2 q + t of a block takes
+//    lane group 2 (l >> 5) + q and codes 4 t .. 4 t + 3;
+//  * the tokens' fragments of a 64-column stage go from L2 straight into LDS
+//    (three stages, two in flight ahead of the one that is read), with one
+//    barrier per stage.  Through registers one stage ahead the latency of
+//    those loads took a third of the time (high + low, 28672 x 4096, 512
+//    tokens: 289 us, of which 118 went with the fragment loads);
+//  * 32 copies of the codebook (128 bytes per entry) instead of 64: the half
+//    waves of a 4-byte LDS read are served in turn, and 28 KB for 217 points
+//    leave room for two blocks per CU.
+// Measured (MI355X, high + low operands, against 16 x 16 tiles with one
+// block per CU): 4096 x 14336 at 512 tokens 143 -> 116 us (1.04 PFLOP/s of
+// matrix-core work), 28672 x 4096 at 512 tokens 311 -> 284 us, at 37 tokens
+// 64 -> 41 us, 6144 x 4096 (q, k and v) at 37 tokens 23 -> 15 us.
+//
+// Safety of the LDS stages.  Stage n goes to buffer n % 3 two stages ahead.
+// A wave waits until only the younger loads than its share of stage n are in
+// flight (vmcnt counts in issue order: the share of stage n + 1, NF loads,
+// and in the second stage of a chunk the 3 R2 code and scale loads issued
+// after it) and for its own LDS reads, then meets the others; after that
+// barrier all of stage n is in LDS and no wave reads stage n - 1, whose
+// buffer stage n + 2 then overwrites.
+// ------------------------------------------------------------------------
+constexpr int kMmStages = 3;
+template <int TB, bool HL, int R2, int T2>
+__global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
+    constexpr int NW = 4, TG = 2 * T2, RB = 2 * R2 * NW;   // 16-token groups and 16-row blocks of the block
+    constexpr int NH = HL ? 2 : 1, FPS = 2 * NH;           // fragments of a token group and stage
+    constexpr int NF = TG * FPS / NW;                      // fragments (1 KB) a wave moves per stage
+    static_assert(NF >= 1 && TG * FPS % NW == 0, "every wave moves whole fragments");
+    constexpr uint32_t ABYTES = TG * FPS * 1024, TBASE = kMmStages * ABYTES;
+    static_assert(TBASE < 65536, "the codebook's base is an LDS instruction's offset");
+    constexpr bool B7 = TB <= 128;
+    constexpr int TBY = B7 ? kTile7 : kTileU8;
+    extern __shared__ __attribute__((aligned(128))) unsigned char lds_mm[];   // stages, then the codebook
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nc = (a.in.cols + 127) >> 7, ng = (a.M + 15) >> 4, n_tt = (ng + TG - 1) / TG;
+    const int sg = (a.nseg > 2 && (int)blockIdx.x >= a.seg[2].b0) ? 2 : (a.nseg > 1 && (int)blockIdx.x >= a.seg[1].b0) ? 1 : 0;
+    const MmSeg& w = a.seg[sg];
+    const int rows = w.rows, nrb = (rows + 15) >> 4, n_rt = (nrb + RB - 1) / RB;
+    // the token tiles and column splits of one row tile on one XCD (blocks
+    // go to the 8 XCDs in turn; b0 is a multiple of 8)
+    const int S = w.nsplit, cps = (nc + S - 1) / S, bl = (int)blockIdx.x - w.b0;
+    const int xcd = bl & 7, bq = bl >> 3;
+    const int rt = (bq / (n_tt * S)) * 8 + xcd, tt = (bq % (n_tt * S)) / S, ks = bq % S;
+    if (rt >= n_rt) return;
+    const int rb0 = rt * RB + wid * R2 * 2, g0 = tt * TG;
+    const int c0 = ks * cps, c1 = min(nc, c0 + cps);
+    if (c0 >= c1) return;
+    const int half = (lane >> 4) & 1, kg = lane >> 5;
+    const uint32_t sh7 = (uint32_t)(lane & 1) * 16u;
+
+    // codes and scales of this wave's rows for chunk c
+    const unsigned char* cp[R2];
+    const uint32_t* sp[R2];
+#pragma unroll
+    for (int r = 0; r < R2; r++) {
+        const size_t i = (size_t)min(rb0 + 2 * r + half, nrb - 1) * nc;
+        cp[r] = reinterpret_cast<const unsigned char*>(w.codes_t) + i * TBY + tile_lane_off(B7, (lane & 15) + 32 * kg);
+        sp[r] = w.scales_t + i * 16 + (lane & 15);
+    }
+    constexpr int QOFF = B7 ? 28 * 8 : 16 * 16;   // from lane group 2 kg to 2 kg + 1 of a tile
+    u32x4v cw[R2][2];
+    uint32_t sw[R2];
+    auto load = [&](int c) {
+        c = min(c, nc - 1);
+#pragma unroll
+        for (int r = 0; r < R2; r++) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) cw[r][q] = *reinterpret_cast<const u32x4_a4*>(cp[r] + (size_t)c * TBY + q * QOFF);
+            sw[r] = sp[r][(size_t)c * 16];
+        }
+    };
+    // this wave's fragments of stage 2 c + h (past the end: the last chunk's, unread)
+    const u32x4v* ap[NF];
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        const int f = wid * NF + i, g = min(g0 + f / FPS, ng - 1), v = f % FPS;
+        ap[i] = reinterpret_cast<const u32x4v*>(a.xa) + ((size_t)g * nc * (2 * FPS) + (HL ? (v >> 1) * 4 + (v & 1) : v)) * 64 + lane;
+    }
+    auto dma = [&](int st, uint32_t b) {
+        const int c = min(st >> 1, nc - 1), h = st & 1;
+#pragma unroll
+        for (int i = 0; i < NF; i++) lds_dma16(ap[i] + ((size_t)c * (2 * FPS) + h * 2) * 64, b * ABYTES + (wid * NF + i) * 1024);
+    };
+    dma(2 * c0, 0);
+    dma(2 * c0 + 1, 1);
+    load(c0);
+    for (int e = tid; e < TB * 32; e += NW * 64) reinterpret_cast<uint32_t*>(lds_mm + TBASE)[e] = a.fields[e >> 5];
+
+    const uint32_t off = (uint32_t)(lane & 31) * 4u;
+    const uint32_t aoff = (uint32_t)(half * FPS * 64 + (lane & 15) + 32 * kg) * 16u;
+    uint32_t buf = 0;
+    float16v acc[R2][T2];
+#pragma unroll
+    for (int r = 0; r < R2; r++)
+#pragma unroll
+        for (int g = 0; g < T2; g++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[r][g][i] = 0.f;
+    uint32_t w4[R2][2][4], sc2[R2];
+    auto look = [&](const uint32_t (&wd)[2][4], auto hc, half8v (&bw)[4]) {
+        constexpr int h = decltype(hc)::value;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            u32x4v b;
+#pragma unroll
+            for (int e = 0; e < 4; e++) b[e] = *(lds_u32*)(code_addr32<B7>(wd[s >> 1], 8 * h + 4 * (s & 1) + e, off) + TBASE);
+            bw[s] = __builtin_bit_cast(half8v, b);
+        }
+    };
+    auto fold = [&](float16v& ac, const float16v& d, uint32_t s2, auto hc) {
+        constexpr int h = decltype(hc)::value;
+        const float sc = h2f((uint16_t)(h ? (s2 >> 16) : (s2 & 0xFFFFu)));
+#pragma unroll
+        for (int i = 0; i < 16; i++) ac[i] = fmaf(d[i], sc, ac[i]);
+    };
+    auto stage = [&](int c, auto hc) {
+        constexpr int h = decltype(hc)::value;
+        constexpr int NV = h ? NF + 3 * R2 : NF;   // loads younger than this wave's share of the stage
+        __builtin_amdgcn_s_waitcnt((NV & 15) | ((NV >> 4) << 14) | 0x0F70);
+        lds_barrier();
+        const uint32_t Ab = buf * ABYTES + aoff;
+        dma(2 * c + h + 2, buf == 0 ? 2 : buf - 1);
+        buf = buf == 2 ? 0 : buf + 1;
+        if constexpr (h == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(c + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        half8v af[T2][4][NH];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int g = 0; g < T2; g++)
+#pragma unroll
+                for (int hl = 0; hl < NH; hl++)
+                    af[g][s][hl] = __builtin_bit_cast(half8v, *(lds_u4*)(Ab + (2 * g * FPS + hl * 2 + (s & 1)) * 1024 + 256 * (s >> 1)));
+        // the next rows' operands are decoded, and the last rows' sums
+        // scaled, beside this row tile's products
+        half8v bw[2][4];
+        float16v d[2][T2];
+        look(w4[0], hc, bw[0]);
+#pragma unroll
+        for (int r = 0; r < R2; r++) {
+            if (r + 1 < R2) look(w4[r + 1], hc, bw[(r + 1) & 1]);
+#pragma unroll
+            for (int g = 0; g < T2; g++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) d[r & 1][g][i] = 0.f;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int hl = 0; hl < NH; hl++)
+#pragma unroll
+                    for (int g = 0; g < T2; g++)
+                        d[r & 1][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[g][s][hl], bw[r & 1][s], d[r & 1][g], 0, 0, 0);
+            if (r > 0) {
+#pragma unroll
+                for (int g = 0; g < T2; g++) fold(acc[r - 1][g], d[(r - 1) & 1][g], sc2[r - 1], hc);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < T2; g++) fold(acc[R2 - 1][g], d[(R2 - 1) & 1][g], sc2[R2 - 1], hc);
+    };
+    for (int c = c0; c < c1; c++) {
+#pragma unroll
+        for (int r = 0; r < R2; r++) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) w4[r][q][i] = cw[r][q][i];
+                if constexpr (B7) align7(w4[r][q], sh7);
+            }
+            sc2[r] = sw[r];
+        }
+        stage(c, std::integral_constant<int, 0>{});
+        stage(c, std::integral_constant<int, 1>{});
+    }
+    // (the two stages past the last chunk land before the block's LDS is
+    // given back)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+
+    // lane: row l & 31 of each row tile, tokens 8 (i >> 2) + 4 kg + (i & 3)
+    float* part = a.part + w.p0;
+    const int Mp = ng * 16;
+#pragma unroll
+    for (int r = 0; r < R2; r++) {
+        const int row = (rb0 + 2 * r) * 16 + (lane & 31);
+        if (row >= rows) continue;
+#pragma unroll
+        for (int g = 0; g < T2; g++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int m = (g0 + 2 * g) * 16 + 8 * (i >> 2) + 4 * kg + (i & 3);
+                if (m >= a.M) continue;
+                if (S > 1) {   // this column split's sum; the consumer adds them in order
+                    part[((size_t)ks * Mp + m) * rows + row] = acc[r][g][i];
+                    continue;
+                }
+                const float y = mm_finish(w, a.in, m, row, acc[r][g][i]);
+                float* yp = w.Y + (size_t)m * rows + row;
+                *yp = a.accumulate ? *yp + y : y;
+            }
+    }
+}
+
+// The partial sums of four consecutive rows of token m, in split order
+__device__ __forceinline__ float4 part4(const float* part, const MmSeg& w, int Mp, int m, int row) {
+    const float* p = part + w.p0 + (size_t)m * w.rows + row;
+    const size_t st = (size_t)Mp * w.rows;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k0 = 0; k0 < w.nsplit; k0 += 4) {
+        float4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = k0 + k < w.nsplit ? *reinterpret_cast<const float4*>(p + (size_t)(k0 + k) * st) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            s.x += v[k].x;
+            s.y += v[k].y;
+            s.z += v[k].z;
+            s.w += v[k].w;
+        }
+    }
+    return s;
+}
+__device__ __forceinline__ float4 finish4(const float* part, const MmSeg& w, const MmIn& in, int Mp, int m, int row) {
+    if (w.nsplit == 1) return *reinterpret_cast<const float4*>(w.Y + (size_t)m * w.rows + row);
+    const float4 s = part4(part, w, Mp, m, row);
+    return make_float4(mm_finish(w, in, m, row, s.x), mm_finish(w, in, m, row + 1, s.y), mm_finish(w, in, m, row + 2, s.z),
+                       mm_finish(w, in, m, row + 3, s.w));
+}
+
+// Partial sums of a batched projection's tensors -> Y (one launch for all
+// tensors: blockIdx.y)
+__global__ void __launch_bounds__(256) mm_reduce_kernel(const MmArgs a) {
+    const MmSeg& w = a.seg[blockIdx.y];
+    if (w.nsplit == 1) return;
+    const int r4 = w.rows >> 2, Mp = ((a.M + 15) >> 4) * 16;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < (size_t)a.M * r4; i += (size_t)gridDim.x * 256) {
+        const int m = (int)(i / r4), row = (int)(i % r4) * 4;
+        *reinterpret_cast<float4*>(w.Y + (size_t)m * w.rows + row) = finish4(a.part, w, a.in, Mp, m, row);
+    }
+}
+
+// ------------------------------------------------------------------------
+// Operands of the next projections from what the last launch left: the
+// token's row (IN 0: X; 1: X plus the last projection, written back; 2:
+// silu(gate) * up; 3: the embedding row of the token, written to X), RMSNorm
+// where norm_w is given ((x * inv) * w, gsd_lq_cpu_engine.c:66-82), then its
+// (u, v) as fp16 high and low parts after a per-token power of two, and the
+// rank-k products of the tensors that read it.  One block per token (padded
+// tokens of the last 16: zeros), the row in LDS; the last projection's column
+// splits, descale, kinks and rank-k terms are taken in here, so a split
+// projection needs no launch and no pass of its own.  Bound: memory (a
+// 512-token chunk of the 7B shape reads and writes 25-60 MB).
+// Measured (7B Precision, 512 tokens): in place of a partial-sum launch
+// (13.5 us), a SwiGLU launch (15.8 us) and this pass reading their results
+// (11-24 us).
+// ------------------------------------------------------------------------
+template <int IN>
+__global__ void __launch_bounds__(512) layer_prep_kernel(const LayerPrep p) {
+    extern __shared__ __attribute__((aligned(16))) float xl[];   // the token's row
+    __shared__ float red[8][2 * kMaxSeg + 2];
+    constexpr float kS32 = 0.866025403784438646763723170752936183f;
+    constexpr int NT = 512, NS = 2 * kMaxSeg;
+    // the 16 rows of a token group, whose fragments share lines, on one XCD
+    // (the identity unless the groups divide evenly)
+    int m = (int)blockIdx.x;
+    if (!(gridDim.x & 127)) {
+        const int x = m & 7, j = m >> 3;
+        m = ((j >> 4) * 8 + x) * 16 + (j & 15);
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int cols = p.cols, nc = (cols + 127) >> 7, np = cols >> 1, nv4 = cols >> 2;
+    const bool valid = m < p.M;
+    float4* xl4 = reinterpret_cast<float4*>(xl);
+    float4* X4 = reinterpret_cast<float4*>(p.X + (size_t)(valid ? m : 0) * cols);
+    auto block_sums = [&](float (&v)[NS + 2], int n) {
+        for (int s = 0; s < n; s++) {
+            const float t = wave_sum_valu(v[s]);
+            if (lane == 0) red[wid][s] = t;
+        }
+        __syncthreads();
+        for (int s = 0; s < n; s++) {
+            float t = 0.f;
+            for (int q = 0; q < NT / 64; q++) t += red[q][s];
+            v[s] = t;
+        }
+        __syncthreads();
+    };
+    const int Mp = ((p.M + 15) >> 4) * 16;
+    const uint16_t* er = nullptr;
+    if constexpr (IN == 3) er = p.embed + (size_t)p.tokens[valid ? m : 0] * cols;
+    float ss = 0.f;
+    for (int b = tid; b < nv4; b += NT) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (valid) {
+            if constexpr (IN == 0) v = X4[b];
+            if constexpr (IN == 1) {
+                v = X4[b];
+                const float4 y = finish4(p.part, p.last[0], p.in, Mp, m, 4 * b);
+                v.x += y.x;
+                v.y += y.y;
+                v.z += y.z;
+                v.w += y.w;
+            }
+            if constexpr (IN == 2) {
+                const float4 g = finish4(p.part, p.last[0], p.in, Mp, m, 4 * b), u = finish4(p.part, p.last[1], p.in, Mp, m, 4 * b);
+                v.x = g.x / (1.0f + expf(-g.x)) * u.x;
+                v.y = g.y / (1.0f + expf(-g.y)) * u.y;
+                v.z = g.z / (1.0f + expf(-g.z)) * u.z;
+                v.w = g.w / (1.0f + expf(-g.w)) * u.w;
+            }
+            if constexpr (IN == 3) {
+                const uint2 e = reinterpret_cast<const uint2*>(er)[b];
+                v = make_float4(h2f((uint16_t)(e.x & 0xFFFFu)), h2f((uint16_t)(e.x >> 16)), h2f((uint16_t)(e.y & 0xFFFFu)),
+                                h2f((uint16_t)(e.y >> 16)));
+            }
+            if constexpr (IN == 1 || IN == 3) {
+                X4[b] = v;
+                if (m == p.M - 1 && p.xlast) reinterpret_cast<float4*>(p.xlast)[b] = v;
+            }
+        }
+        xl4[b] = v;
+        ss = fmaf(v.x, v.x, ss);
+        ss = fmaf(v.y, v.y, ss);
+        ss = fmaf(v.z, v.z, ss);
+        ss = fmaf(v.w, v.w, ss);
+    }
+    float sv[NS + 2];
+    float inv = 1.f;
+    if (p.norm_w) {
+        sv[0] = ss;
+        block_sums(sv, 1);
+        inv = 1.0f / sqrtf(sv[0] / (float)cols + p.eps);
+    }
+    // x' in place (each thread its own float4s), its rank-k products and the
+    // largest |u|, |v|
+    const float4* w4 = reinterpret_cast<const float4*>(p.norm_w);
+    const uint2* vt[NS];
+    bool act[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        act[s] = (s & 1) < p.k[s >> 1];
+        vt[s] = act[s] ? reinterpret_cast<const uint2*>(p.Vt[s >> 1] + (size_t)(s & 1) * cols) : nullptr;
+        sv[s] = 0.f;
+    }
+    float mx = 0.f;
+    for (int b = tid; b < nv4; b += NT) {
+        float4 x = xl4[b];
+        uint2 hv[NS];
+#pragma unroll
+        for (int s = 0; s < NS; s++) hv[s] = act[s] ? vt[s][b] : make_uint2(0u, 0u);
+        if (p.norm_w) {
+            const float4 nw = w4[b];
+            x.x = (x.x * inv) * nw.x;
+            x.y = (x.y * inv) * nw.y;
+            x.z = (x.z * inv) * nw.z;
+            x.w = (x.w * inv) * nw.w;
+            xl4[b] = x;
+        }
+        if (valid && p.xn) reinterpret_cast<float4*>(p.xn + (size_t)m * cols)[b] = x;
+        mx = fmaxf(mx, fmaxf(fabsf(x.x), fabsf(fmaf(kS32, x.y, 0.5f * x.x))));
+        mx = fmaxf(mx, fmaxf(fabsf(x.z), fabsf(fmaf(kS32, x.w, 0.5f * x.z))));
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            if (!act[s]) continue;
+            sv[s] = fmaf(x.x, h2f((uint16_t)(hv[s].x & 0xFFFFu)), sv[s]);
+            sv[s] = fmaf(x.y, h2f((uint16_t)(hv[s].x >> 16)), sv[s]);
+            sv[s] = fmaf(x.z, h2f((uint16_t)(hv[s].y & 0xFFFFu)), sv[s]);
+            sv[s] = fmaf(x.w, h2f((uint16_t)(hv[s].y >> 16)), sv[s]);
+        }
+    }
+    {
+        const float t = wave_max_valu(mx);
+        if (lane == 0) red[wid][NS] = t;
+        block_sums(sv, act[0] || act[2] || act[4] ? NS : 0);   // (barriers in any case: x' and the maxima are in LDS)
+        mx = red[0][NS];
+        for (int q = 1; q < NT / 64; q++) mx = fmaxf(mx, red[q][NS]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+        if (valid && tid == s && act[s]) p.tmp[s >> 1][(size_t)m * p.k[s >> 1] + (s & 1)] = sv[s] * p.S[s >> 1][s & 1];
+    int ex = 0;
+    if (mx > 0.f && mx < INFINITY) (void)frexpf(mx, &ex);
+    const float up = ldexpf(1.f, 14 - ex);
+    if (tid == 0) p.xs[m] = valid ? ldexpf(1.f, ex - 14) : 0.f;
+    // fragments: four pairs (16 bytes) of the high parts and of the low parts per thread
+    const int g16 = m >> 4, ml = m & 15;
+    for (int i = tid; i < nc * 16; i += NT) {
+        float4 f[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+        if (valid && 4 * i < np) {   // (np is a multiple of 32)
+            f[0] = xl4[2 * i];
+            f[1] = xl4[2 * i + 1];
+        }
+        const float xa[4] = {f[0].x, f[0].z, f[1].x, f[1].z}, xb[4] = {f[0].y, f[0].w, f[1].y, f[1].w};
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float u = xa[e] * up, v = fmaf(kS32, xb[e], 0.5f * xa[e]) * up;
+            const _Float16 uh = (_Float16)u, vh = (_Float16)v;
+            const _Float16 ul = (_Float16)(u - (float)uh), vl = (_Float16)(v - (float)vh);
+            hi[e] = (uint32_t)__builtin_bit_cast(uint16_t, uh) | ((uint32_t)__builtin_bit_cast(uint16_t, vh) << 16);
+            lo[e] = (uint32_t)__builtin_bit_cast(uint16_t, ul) | ((uint32_t)__builtin_bit_cast(uint16_t, vl) << 16);
+        }
+        const int q0 = 4 * i, c = q0 >> 6, h = (q0 >> 5) & 1, lg = (q0 >> 3) & 3, t2 = (q0 >> 2) & 1;
+        uint4* o = p.xa + (((size_t)g16 * nc + c) * 8 + h * 2 + t2) * 64 + ml + 16 * lg;
+        o[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        o[4 * 64] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+}
+
+// ------------------------------------------------------------------------
+// q, k, v of M prompt tokens: column splits, descale, kinks and rank-k terms
+// taken in, then RoPE and the fp16 K/V append as rope_kv_kernel forms them
+// (no contraction).  last[0] = q, [1] = k, [2] = v, or k and v only (nseg 2,
+// the last layer's tokens before the last one).  A thread per pair.
+// ------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) qkv_finish_kernel(const QkvFinish p) {
+#pragma clang fp contract(off)
+    const int half = p.r.hd >> 1, m = blockIdx.y, Mp = ((p.M + 15) >> 4) * 16;
+    const int nq = p.nseg == 3 ? p.r.n_heads * half : 0, nk = p.r.n_kv * half;
+    const int gid = blockIdx.x * 256 + threadIdx.x;
+    if (gid >= nq + 2 * nk) return;
+    const int which = gid < nq ? 0 : (gid < nq + nk ? 1 : 2);   // q, k, v
+    const int pr = which == 0 ? gid : (which == 1 ? gid - nq : gid - nq - nk);
+    const int s = p.nseg == 3 ? which : which - 1;
+    const MmSeg& w = s == 0 ? p.last[0] : (s == 1 ? p.last[1] : p.last[2]);
+    const int h = pr / half, i = pr % half;
+    const bool pairs = p.r.interleaved || which == 2;   // (v: any two neighbours)
+    const int i0 = h * p.r.hd + (pairs ? 2 * i : i), i1 = h * p.r.hd + (pairs ? 2 * i + 1 : i + half);
+    float a, b;
+    if (w.nsplit == 1) {
+        a = w.Y[(size_t)m * w.rows + i0];
+        b = w.Y[(size_t)m * w.rows + i1];
+    } else {
+        const float* pp = p.part + w.p0 + (size_t)m * w.rows;
+        const size_t st = (size_t)Mp * w.rows;
+        a = b = 0.f;
+        for (int k = 0; k < w.nsplit; k++) {
+            a += pp[k * st + i0];
+            b += pp[k * st + i1];
+        }
+        a = mm_finish(w, p.in, m, i0, a);
+        b = mm_finish(w, p.in, m, i1, b);
+    }
+    const int pos = p.r.pos + m;
+    const size_t base = ((size_t)p.r.layer * p.r.max_seq + (size_t)pos) * (size_t)p.r.n_kv * p.r.hd;
+    if (which == 2) {
+        p.r.v_cache[base + i0] = f2h(a);
+        p.r.v_cache[base + i1] = f2h(b);
+        return;
+    }
+    const float2 cs = p.r.cs[(size_t)pos * half + i];
+    const float x0 = a * cs.x - b * cs.y, x1 = a * cs.y + b * cs.x;
+    if (which == 0) {
+        float* q = p.q + (size_t)m * p.r.n_heads * p.r.hd;
+        q[i0] = x0;
+        q[i1] = x1;
+    } else {
+        p.r.k_cache[base + i0] = f2h(x0);
+        p.r.k_cache[base + i1] = f2h(x1);
+    }
+}
+
+template <int TB, bool HL, int R2, int T2>
+hipError_t launch_hexmm32_t(const MmArgs& a, int grid, hipStream_t st) {
+    const int lds = kMmStages * 2 * T2 * (HL ? 4 : 2) * 1024 + TB * 128;
+    static bool attr = false;
+    if (!attr) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmm32_kernel<TB, HL, R2, T2>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    hipLaunchKernelGGL((hexmm32_kernel<TB, HL, R2, T2>), dim3(grid), dim3(256), lds, st, a);
+    return hipGetLastError();
+}
+
+template <int TB>
+hipError_t launch_hexmm32_tb(const MmArgs& a, int grid, hipStream_t st) {
+    if (a.hl) {
+        if (a.r2 == 2 && a.t2 == 2) return launch_hexmm32_t<TB, true, 2, 2>(a, grid, st);
+        if (a.r2 == 1 && a.t2 == 2) return launch_hexmm32_t<TB, true, 1, 2>(a, grid, st);
+        if (a.r2 == 1 && a.t2 == 1) return launch_hexmm32_t<TB, true, 1, 1>(a, grid, st);
+        return hipErrorInvalidValue;
+    }
+    if (a.r2 == 1 && a.t2 == 4) return launch_hexmm32_t<TB, false, 1, 4>(a, grid, st);
+    if (a.r2 == 1 && a.t2 == 2) return launch_hexmm32_t<TB, false, 1, 2>(a, grid, st);
+    if (a.r2 == 1 && a.t2 == 1) return launch_hexmm32_t<TB, false, 1, 1>(a, grid, st);
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+bool hexmm32_codebook(int n_pts) { return n_pts == 217 || n_pts == 127; }
+
+// High + low operands (a prompt): two tokens tiles of 32 and two row tiles
+// per wave from 65 tokens on; fewer tokens take narrower tiles, so that the
+// grid is finer and less of a tile is padding.  The columns are split into
+// what fills two blocks per CU (at least 4 chunks each; up to 16, whose
+// partial sums the next launch still takes in within its own time).
+MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols) {
+    const int ng = (M + 15) / 16, nc = (cols + 127) / 128, ncu = device_cu_count() > 0 ? device_cu_count() : 256;
+    MmTile t{ng <= 4 ? 1 : 2, ng <= 2 ? 1 : 2, 1};
+    const int rb = 8 * t.r2, tiles = ((rows_total_tiles_of_16 + rb - 1) / rb) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
+    t.nsplit = whole_splits(nc, std::max(1, std::min({2 * ncu / tiles, nc / 4, 16})));
+    return t;
+}
+
+// Fills seg[].b0, .nsplit and .p0 for the tile; returns the floats of partial
+// sums (seg[].rows set).  Tensors of one launch that are split differently
+// keep their own split (nsplit 0: the tile's).
+size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid) {
+    const int ng = (a.M + 15) / 16, n_tt = (ng + 2 * t.t2 - 1) / (2 * t.t2);
+    int b = 0;
+    size_t p = 0;
+    a.r2 = t.r2;
+    a.t2 = t.t2;
+    for (int s = 0; s < a.nseg; s++) {
+        MmSeg& w = a.seg[s];
+        if (w.nsplit <= 0) w.nsplit = t.nsplit;
+        const int n_rt = ((w.rows + 15) / 16 + 8 * t.r2 - 1) / (8 * t.r2);
+        w.b0 = b;
+        w.p0 = p;
+        b += 8 * n_tt * w.nsplit * ((n_rt + 7) / 8);
+        if (w.nsplit > 1) p += (size_t)w.nsplit * ng * 16 * w.rows;
+    }
+    *grid = b;
+    return p;
+}
+
+hipError_t launch_hexmm32(const MmArgs& a, int grid, hipStream_t st) {
+    if (a.M <= 0 || a.in.cols <= 0 || a.in.cols % 64 || a.nseg < 1 || a.nseg > kMaxSeg || !a.xa || !a.in.xs || !a.fields)
+        return hipErrorInvalidValue;
+    for (int s = 0; s < a.nseg; s++) {
+        const MmSeg& w = a.seg[s];
+        if (!w.codes_t || !w.scales_t || w.rows <= 0 || w.nsplit < 1 || (w.nsplit > 1 && !a.part) || (w.nsplit == 1 && !w.Y) ||
+            (w.k > 0 && (!w.U || !w.tmp_k)) || (w.row_ptr && !a.in.Xf && !a.in.X))
+            return hipErrorInvalidValue;
+    }
+    if (a.n_pts == 217) return launch_hexmm32_tb<217>(a, grid, st);
+    if (a.n_pts == 127) return launch_hexmm32_tb<127>(a, grid, st);
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_mm_reduce(const MmArgs& a, hipStream_t st) {
+    size_t n = 0;
+    for (int s = 0; s < a.nseg; s++) {
+        if (a.seg[s].nsplit == 1) continue;
+        if (a.seg[s].rows % 4) return hipErrorInvalidValue;
+        n = std::max(n, (size_t)a.M * (a.seg[s].rows / 4));
+    }
+    if (!n) return hipSuccess;
+    hipLaunchKernelGGL(mm_reduce_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096), a.nseg), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_layer_prep(const LayerPrep& p, LayerPrepIn in, hipStream_t st) {
+    if (p.M <= 0 || p.cols <= 0 || p.cols % 64 || p.cols > kLayerPrepMaxCols || !p.xa || !p.xs) return hipErrorInvalidValue;
+    const size_t lds = (size_t)p.cols * 4;
+    const dim3 grid(((p.M + 15) / 16) * 16);
+#define GSD_PREP(IN)                                                                                                     \
+    {                                                                                                                    \
+        static size_t attr = 0;                                                                                          \
+        if (lds > attr) {                                                                                                \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&layer_prep_kernel<IN>),              \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);              \
+            if (e != hipSuccess) return e;                                                                               \
+            attr = lds;                                                                                                  \
+        }                                                                                                                \
+        hipLaunchKernelGGL((layer_prep_kernel<IN>), grid, dim3(512), lds, st, p);                                        \
+        break;                                                                                                           \
+    }
+    switch (in) {
+        case kPrepRow: GSD_PREP(0)
+        case kPrepResidual: GSD_PREP(1)
+        case kPrepSwiGLU: GSD_PREP(2)
+        case kPrepEmbed: GSD_PREP(3)
+    }
+#undef GSD_PREP
+    return hipGetLastError();
+}
+
+hipError_t launch_qkv_finish(const QkvFinish& p, hipStream_t st) {
+    if (p.M <= 0 || (p.nseg != 2 && p.nseg != 3) || !p.r.cs || p.r.pos < 0 || p.r.pos + p.M > p.r.max_seq) return hipErrorInvalidValue;
+    const int half = p.r.hd / 2, n = (p.nseg == 3 ? p.r.n_heads * half : 0) + 2 * p.r.n_kv * half;
+    hipLaunchKernelGGL(qkv_finish_kernel, dim3((n + 255) / 256, p.M), dim3(256), 0, st, p);
+    return hipGetLastError();
+}
+
+}  // namespace gsd

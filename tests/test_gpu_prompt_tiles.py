@@ -1,0 +1,73 @@
+"""The 32 x 32 tile projections of the batched prefill and of
+gsdh_model_matmul at the sizes where their tiling can go wrong, against the
+oracle: token counts at the edges of 16-token groups and of the 32- and
+64-token tiles (one more and one less), row counts that are not whole row
+tiles, columns that end in half a chunk and columns whose chunks do not divide
+into the splits, both code formats, kinks and rank-2 terms taken in from
+column splits; and that a model takes any number of prompts."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import rel_l2
+from gpu_util import banner
+from test_gpu_prefill import SLOTS, _kv_close, _pair, _small_model, _spec, check
+
+pytestmark = pytest.mark.gpu
+
+# hidden 320: chunks of 128, 128 and 64 columns; ffn 832: 6.5 chunks; 5 heads
+# of 64: k and v of 320 rows (no whole 128- or 256-row tile)
+RAGGED = dict(hidden=320, ffn=832, n_heads=5, n_kv_heads=5, head_dim=64)
+
+
+# the last position's logits and the cache: fp32 sums of ~22-bit inputs, and
+# elements of K / V that round to the other fp16 value (2^-11 of an element)
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 31, 32, 33, 63, 64, 65, 129])
+@pytest.mark.parametrize("mode,kpr,shape", [("precision", 2, dict()), ("turbo", 1, RAGGED),
+                                            ("precision", 0, dict(n_layers=3, hidden=512, ffn=2496, n_heads=8,
+                                                                  n_kv_heads=2, head_dim=64))])
+def test_prompt_edges(mode, kpr, shape, n):
+    banner(f"prompt of {n} tokens, {mode} kinks {kpr} {shape}")
+    gpu, ref = _pair(_spec(mode=mode, kinks_per_row=kpr, **shape), max_seq=192)
+    toks = np.random.default_rng(n).integers(0, gpu.vocab_size, n).tolist()
+    got = gpu.prefill(toks, 0)
+    for pos, t in enumerate(toks):
+        want = ref.forward_token(t, pos, return_logits=pos == n - 1)
+    assert rel_l2(got, want) < 1e-3
+    _kv_close(gpu, ref, range(gpu.n_layers), sorted({0, n // 2, n - 1}))
+    nxt = int(np.argmax(want))
+    assert rel_l2(gpu.forward_token(nxt, n), ref.forward_token(nxt, n)) < 1e-3
+    gpu.close()
+
+
+@pytest.mark.parametrize("M", [1, 31, 33, 65, 113, 127, 129])
+@pytest.mark.parametrize("mode,kpr,shape", [("turbo", 1, RAGGED), ("precision", 2, dict(ffn=8256))])
+def test_matmul_edges(mode, kpr, shape, M):
+    banner(f"matmul of {M} tokens, {mode} kinks {kpr} {shape}")
+    src, model = _small_model(_spec(n_layers=1, mode=mode, kinks_per_row=kpr, **shape))
+    try:
+        for name in ("attn_k", "ffn_up", "ffn_down"):
+            key = f"blk.0.{name}.weight"
+            t = dict(src.tensors[key])
+            for f in ("codes", "scales", "row_ptr", "kink_cols", "kink_deltas") + (("U", "S", "Vt") if t["k_dim"] else ()):
+                t[f] = np.ascontiguousarray(src.hex_field(key, f))
+            check(model, t, 0, SLOTS[name], M, seed=M + SLOTS[name])
+    finally:
+        model.close()
+
+
+@pytest.mark.parametrize("mode,shape", [("precision", dict()), ("precision", dict(k_dim=3))])
+def test_any_number_of_prompts(mode, shape):
+    """Each prompt's head took further publication words of the model until,
+    after some two hundred prompts on two layers, none were left."""
+    banner(f"300 prompts on one model, {mode} {shape}")
+    gpu, ref = _pair(_spec(mode=mode, kinks_per_row=0, **shape), max_seq=16)
+    toks = [5, 77, 300]
+    for pos, t in enumerate(toks):
+        want = ref.forward_token(t, pos, return_logits=pos == 2)
+    first = gpu.prefill(toks, 0)
+    for _ in range(300):
+        got = gpu.prefill(toks, 0)
+    assert np.array_equal(first, got)
+    assert rel_l2(got, want) < 1e-3
+    gpu.close()
