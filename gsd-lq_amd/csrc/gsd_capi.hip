@@ -991,11 +991,32 @@ int issue_prefill(gsdh_model* m, int M, int p0) {
     return 0;
 }
 
+// One decode layer without the fused attention: the step's q/k/v, attention
+// and o + FFN launches for x at the step position.
+int issue_layer(gsdh_model* m, int l) {
+    const auto& c = m->c;
+    int rc = issue_linear(m, l, 1);
+    if (rc) return rc;
+    if (!c.rope_interleaved) {   // (i, i+hd/2) pairs are not adjacent rows: separate kernel
+        RopeKV r{};
+        r.cs = m->cs; r.pos_dev = &m->st->pos; r.k_cache = m->kc; r.v_cache = m->vc; r.layer = l;
+        r.n_heads = c.n_heads; r.n_kv = c.n_kv_heads; r.hd = c.head_dim; r.max_seq = c.max_seq_len;
+        r.interleaved = 0;
+        HIPCHK(launch_rope_kv(m->q, m->k, m->v, r, nullptr, m->stream));
+    }
+    HIPCHK(launch_attention(layer_attention(m, l, 0), m->stream));
+    return issue_linear(m, l, 2 | 4 | 8);
+}
+
 // Prompt tokens P.tok[0..M) at positions p0.. on the 32 x 32 tile
 // projections, what issue_prefill computes: q, k and v in one launch, gate
 // and up in one, and each projection's column splits, descale, kink, rank-k,
 // residual and SwiGLU terms taken in by the pass that prepares the next
-// input.  9 launches per layer instead of 19.  x is then the last token's.
+// input.  9 launches per layer instead of 19.  The last layer forms what its
+// readers need: K and V of every token and, of the last token of the prompt
+// (`last`), the layer itself, by the decode step's launches; x is then the
+// last token's.  (The other tokens' attention, o and FFN of that layer have
+// no reader.)
 int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
     const auto& c = m->c;
     auto& P = m->pf;
@@ -1008,12 +1029,12 @@ int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
     // the input `in` of tensors ts[0..n) prepared, then their projection
     // into Y[i] (added to it with accumulate) or, split, as partial sums
     auto project = [&](LayerPrepIn kind, float* X, const float* norm_w, int cols, const int* slots, int n, int l,
-                       float* const* Y, bool accumulate) -> int {
+                       float* const* Y, bool accumulate, float* xlast) -> int {
         at ^= 1;
         LayerPrep p{};
         p.X = X; p.embed = m->embed; p.tokens = P.tok; p.in = a.in; p.part = P.part;
         for (int s = 0; s < 2 && s < a.nseg; s++) p.last[s] = a.seg[s];
-        p.norm_w = norm_w; p.eps = c.rms_eps; p.M = M; p.cols = cols; p.xa = P.xa; p.xs = xs[at];
+        p.norm_w = norm_w; p.eps = c.rms_eps; p.M = M; p.cols = cols; p.xa = P.xa; p.xs = xs[at]; p.xlast = xlast;
         MmArgs b{};
         b.nseg = n; b.M = M; b.hl = 1; b.accumulate = accumulate; b.xa = P.xa; b.part = P.part;
         b.in.xs = xs[at]; b.in.cols = cols;
@@ -1045,9 +1066,15 @@ int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
     float* const xo[1] = {P.X};
     float* const gu[2] = {P.G, P.U};
     for (int l = 0; l < c.n_layers; l++) {
+        const bool end = l == c.n_layers - 1;
         // (a projection into X that was not split is in X already)
         LayerPrepIn in = l == 0 ? kPrepEmbed : (a.seg[0].nsplit > 1 ? kPrepResidual : kPrepRow);
-        if ((rc = project(in, P.X, m->norm(l, 0), c.hidden, kQkv, 3, l, qkv, false))) return rc;
+        const int first = end ? 1 : 0;
+        if (end && last && in == kPrepRow)
+            HIPCHK(hipMemcpyAsync(m->x, P.X + (size_t)(M - 1) * c.hidden, (size_t)c.hidden * 4, hipMemcpyDeviceToDevice, m->stream));
+        if ((rc = project(in, P.X, m->norm(l, 0), c.hidden, kQkv + first, 3 - first, l, qkv + first, false,
+                          end && last ? m->x : nullptr)))
+            return rc;
         QkvFinish f{};
         for (int s = 0; s < a.nseg; s++) f.last[s] = a.seg[s];
         f.nseg = a.nseg; f.M = M; f.in = a.in; f.part = P.part; f.q = P.Q;
@@ -1055,26 +1082,20 @@ int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
         f.r.n_kv = c.n_kv_heads; f.r.hd = c.head_dim; f.r.max_seq = c.max_seq_len; f.r.interleaved = c.rope_interleaved;
         // (an unsplit projection left q in P.Q: rotated in place)
         HIPCHK(launch_qkv_finish(f, m->stream));
+        if (end) break;
         PrefillAttn pa{};
         pa.q = P.Q; pa.k_cache = m->kc; pa.v_cache = m->vc; pa.out = P.A; pa.layer = l; pa.p0 = p0; pa.M = M;
         pa.n_heads = c.n_heads; pa.n_kv = c.n_kv_heads; pa.hd = c.head_dim; pa.max_seq = c.max_seq_len;
         pa.sm_scale = 1.0f / (float)std::sqrt((double)c.head_dim);
         HIPCHK(launch_prefill_attention(pa, m->stream));
-        if ((rc = project(kPrepRow, P.A, nullptr, qd, kO, 1, l, xo, true))) return rc;
+        if ((rc = project(kPrepRow, P.A, nullptr, qd, kO, 1, l, xo, true, nullptr))) return rc;
         in = a.seg[0].nsplit > 1 ? kPrepResidual : kPrepRow;
-        if ((rc = project(in, P.X, m->norm(l, 1), c.hidden, kGu, 2, l, gu, false))) return rc;
-        if ((rc = project(kPrepSwiGLU, nullptr, nullptr, c.ffn, kDown, 1, l, xo, true))) return rc;
+        if ((rc = project(in, P.X, m->norm(l, 1), c.hidden, kGu, 2, l, gu, false, nullptr))) return rc;
+        if ((rc = project(kPrepSwiGLU, nullptr, nullptr, c.ffn, kDown, 1, l, xo, true, nullptr))) return rc;
     }
     if (!last) return 0;
-    if (a.seg[0].nsplit == 1) {
-        HIPCHK(hipMemcpyAsync(m->x, P.X + (size_t)(M - 1) * c.hidden, (size_t)c.hidden * 4, hipMemcpyDeviceToDevice, m->stream));
-        return 0;
-    }
-    LayerPrep p{};   // the last layer's down, and the last token's row of it
-    p.X = P.X; p.in = a.in; p.part = P.part; p.last[0] = a.seg[0]; p.M = M; p.cols = c.hidden; p.xa = P.xa;
-    p.xs = xs[at ^ 1]; p.xlast = m->x;
-    HIPCHK(launch_layer_prep(p, kPrepResidual, m->stream));
-    return 0;
+    m->pub_next = 0;   // (ranks of at most 2: no publication words are used)
+    return issue_layer(m, c.n_layers - 1);
 }
 
 // Prompt prompt[0..n) at positions start.. in batches of the prefill chunk;
@@ -1086,6 +1107,8 @@ int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
 // chunk's attention reaches the caller.
 int run_prefill(gsdh_model* m, const int* prompt, int n, int start, bool head, int* tok_stage) {
     auto& P = m->pf;
+    // the step state of the last token from the start: the 32 x 32 tile path
+    // runs that token's last layer as a decode step
     HIPCHK(launch_set_step(m->st, prompt[n - 1], start + n - 1, 1, m->stream));
     for (int b0 = 0; b0 < n; b0 += P.chunk) {
         const int M = std::min(P.chunk, n - b0);
