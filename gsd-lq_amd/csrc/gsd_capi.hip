@@ -793,8 +793,9 @@ size_t matmul_ws_need(int M, int rows, int cols) {
     const size_t xs = ((size_t)(M + 15) / 16 * 16 * 4 + 255) / 256 * 256;
     const size_t tk = ((size_t)M * kMaxRank * 4 + 255) / 256 * 256;
     const MatmulPlan plan = hexmm_plan(M, rows, cols);
-    const size_t pt = plan.nsplit > 1 ? (size_t)plan.nsplit * ((M + 15) / 16 * 16) * rows * 4 : 0;
-    return xa + xs + kMaxSeg * tk + pt;
+    const MmTile t = hexmm32_tile(M, rows, cols);   // (its launch holds up to kMaxSeg tensors' partial sums)
+    const size_t n = std::max(plan.nsplit > 1 ? plan.nsplit : 0, t.nsplit > 1 ? kMaxSeg * t.nsplit : 0);
+    return xa + xs + kMaxSeg * tk + n * ((M + 15) / 16 * 16) * rows * 4;
 }
 
 size_t split_part_bytes(int M, int rows, int cols) {   // the prefill's (high + low operands)
@@ -1602,35 +1603,80 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
     const size_t xs = ((size_t)(M + 15) / 16 * 16 * 4 + 255) / 256 * 256;
     const size_t tk = ((size_t)M * kMaxRank * 4 + 255) / 256 * 256;
     char* w = static_cast<char*>(m->mm_ws);
-    // X's operands once for every tensor of the call
-    HIPCHK(launch_hexmm_xprep(X, M, cols, reinterpret_cast<uint4*>(w), reinterpret_cast<float*>(w + xa), m->stream));
+    uint4* xap = reinterpret_cast<uint4*>(w);
+    float* xsp = reinterpret_cast<float*>(w + xa);
+    // (split partials of the tensors in turn, or of one launch's tensors
+    // after each other: stream order keeps the calls apart)
+    float* part = reinterpret_cast<float*>(w + xa + xs + kMaxSeg * tk);
+    // X's operands once for every tensor of the call, with the rank-k
+    // products where one pass covers them
+    MmXprep xp{};
+    xp.X = X; xp.M = M; xp.cols = cols; xp.xa = xap; xp.xs = xsp;
+    float* tmp[kMaxSeg];
+    for (int i = 0; i < n; i++) {
+        tmp[i] = reinterpret_cast<float*>(w + xa + xs + (size_t)i * tk);
+        xp.Vt[i] = ts[i]->Vt; xp.S[i] = ts[i]->Sv; xp.k[i] = ts[i]->k; xp.tmp[i] = tmp[i];
+    }
+    const bool one_pass = mm_xprep_covers(xp);
+    if (one_pass) {
+        HIPCHK(launch_mm_xprep(xp, m->stream));
+    } else {
+        HIPCHK(launch_hexmm_xprep(X, M, cols, xap, xsp, m->stream));
+        for (int i = 0; i < n; i++)
+            if (ts[i]->k > 0)
+                HIPCHK(launch_lowrank_batched(X, ts[i]->Vt, ts[i]->Sv, tmp[i], M, ts[i]->k, cols, m->stream));
+    }
+    // a tensor's tile and splits depend on its own shape alone, so a call's
+    // result does not depend on which tensors share it
+    MmArgs a{};
+    a.M = M; a.xa = xap; a.part = part; a.in.xs = xsp; a.in.X = X; a.in.cols = cols;
+    auto flush = [&]() -> int {
+        if (!a.nseg) return 0;
+        int grid = 0;
+        (void)hexmm32_layout(a, MmTile{a.r2, a.t2, 1}, &grid);
+        HIPCHK(launch_hexmm32(a, grid, m->stream));
+        HIPCHK(launch_mm_reduce(a, m->stream));
+        a.nseg = 0;
+        return 0;
+    };
+    int rc = 0;
     for (int i = 0; i < n; i++) {
         const HexDev& t = *ts[i];
+        const int n_pts = 3 * t.radius * t.radius + 3 * t.radius + 1;
+        const MmTile tile = hexmm32_codebook(n_pts) && (reinterpret_cast<uintptr_t>(Y[i]) & 15) == 0 ? hexmm32_tile(M, t.rows, cols)
+                                                                                                    : MmTile{};
+        if (tile.nsplit > 0) {
+            if (a.nseg && a.n_pts != n_pts && (rc = flush())) return rc;
+            a.n_pts = n_pts; a.fields = m->fields[t.radius]; a.r2 = tile.r2; a.t2 = tile.t2;
+            MmSeg& sg = a.seg[a.nseg++];
+            sg = mm_seg(t, Y[i]);
+            sg.nsplit = tile.nsplit;
+            sg.tmp_k = t.k > 0 ? tmp[i] : nullptr;
+            continue;
+        }
+        if ((rc = flush())) return rc;
         const MatmulPlan plan = hexmm_plan(M, t.rows, t.cols);
-        float* tmp = reinterpret_cast<float*>(w + xa + xs + (size_t)i * tk);
-        MatmulArgs a{};
-        fill_seg(a.w, t, m, nullptr);
-        a.X = X;
-        a.xa = reinterpret_cast<uint4*>(w);
-        a.xs = reinterpret_cast<float*>(w + xa);
-        a.tmp_k = t.k > 0 ? tmp : nullptr;
-        a.Y = Y[i];
-        a.M = M;
-        a.cols = t.cols;
-        a.nsplit = plan.nsplit;
-        a.tg = plan.tg;
-        a.rbw = plan.rbw;
-        a.prepped = 1;
-        // (split partials of the tensors in turn: stream order keeps them apart)
-        a.part = plan.nsplit > 1 ? reinterpret_cast<float*>(w + xa + xs + kMaxSeg * tk) : nullptr;
-        if (t.k > 0) HIPCHK(launch_lowrank_batched(X, t.Vt, t.Sv, tmp, M, t.k, t.cols, m->stream));
-        HIPCHK(launch_hexmm(a, m->stream));
+        MatmulArgs b{};
+        fill_seg(b.w, t, m, nullptr);
+        b.X = X; b.xa = xap; b.xs = xsp;
+        b.tmp_k = t.k > 0 ? tmp[i] : nullptr;
+        b.Y = Y[i]; b.M = M; b.cols = t.cols;
+        b.nsplit = plan.nsplit; b.tg = plan.tg; b.rbw = plan.rbw; b.prepped = 1;
+        b.part = plan.nsplit > 1 ? part : nullptr;
+        HIPCHK(launch_hexmm(b, m->stream));
     }
-    return 0;
+    return flush();
 }
 
 int gsdh_matmul_plan(int M, int rows, int cols, int* tg, int* rbw, int* nsplit) {
     if (M <= 0 || rows <= 0 || cols <= 0 || !tg || !rbw || !nsplit) return fail(-1, "matmul_plan: bad argument");
+    const MmTile t = hexmm32_tile(M, rows, cols);
+    if (t.nsplit > 0) {   // 16-token groups per block, 16-row blocks per wave
+        *tg = 2 * t.t2;
+        *rbw = 2 * t.r2;
+        *nsplit = t.nsplit;
+        return 0;
+    }
     const MatmulPlan p = hexmm_plan(M, rows, cols);
     *tg = p.tg;
     *rbw = p.rbw;

@@ -313,6 +313,21 @@ struct MmTile {
 };
 bool hexmm32_codebook(int n_pts);   // whether launch_hexmm32 covers the codebook
 MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols);
+MmTile hexmm32_tile(int M, int rows, int cols);   // single operands; nsplit 0: not this path
+// Single fp16 operands of bf16 X [M][cols] and the rank-k products (ranks of
+// at most 2) of the tensors that read it
+struct MmXprep {
+    const uint16_t* X;
+    int M, cols;
+    uint4* xa;
+    float* xs;
+    const uint16_t* Vt[kMaxSeg];
+    const float* S[kMaxSeg];
+    int k[kMaxSeg];
+    float* tmp[kMaxSeg];
+};
+bool mm_xprep_covers(const MmXprep& p);   // columns, ranks and alignment
+hipError_t launch_mm_xprep(const MmXprep& p, hipStream_t stream);
 size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid);
 hipError_t launch_hexmm32(const MmArgs& a, int grid, hipStream_t stream);
 // every split tensor's partial sums -> its Y (rows a multiple of 4)

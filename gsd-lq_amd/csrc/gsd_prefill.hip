@@ -536,6 +536,104 @@ __global__ void __launch_bounds__(256) qkv_finish_kernel(const QkvFinish p) {
     }
 }
 
+// ------------------------------------------------------------------------
+// Operands of bf16 tokens (single fp16 parts, as hexmm_xprep2_kernel) and
+// the rank-k products of the tensors that read them, from one pass over X:
+// one block per token (padded tokens: zeros), the row in registers.  A launch
+// per tensor that read X again for its rank-k products took 7.7 us each at
+// 128 tokens x 4096; this one takes 5 with two tensors' products.
+// ------------------------------------------------------------------------
+__global__ void __launch_bounds__(512) mm_xprep_kernel(const MmXprep p) {
+    constexpr int NS = 2 * kMaxSeg;
+    __shared__ float red[8][NS + 1];
+    constexpr float kS32 = 0.866025403784438646763723170752936183f;
+    int m = (int)blockIdx.x;
+    if (!(gridDim.x & 127)) {   // a token group's rows on one XCD
+        const int x = m & 7, j = m >> 3;
+        m = ((j >> 4) * 8 + x) * 16 + (j & 15);
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int nc = (p.cols + 127) >> 7, ng8 = p.cols >> 3;
+    const bool valid = m < p.M;
+    const uint4* xr = reinterpret_cast<const uint4*>(p.X + (size_t)(valid ? m : 0) * p.cols);
+    uint4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = tid + 512 * k;
+        v[k] = valid && i < ng8 ? xr[i] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    float sv[NS];
+    bool act[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        act[s] = (s & 1) < p.k[s >> 1];
+        sv[s] = 0.f;
+    }
+    float mx = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = tid + 512 * k;
+        const uint32_t w4[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        float xa[4], xb[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            xa[e] = __uint_as_float(w4[e] << 16);
+            xb[e] = __uint_as_float(w4[e] & 0xFFFF0000u);
+            mx = fmaxf(mx, fmaxf(fabsf(xa[e]), fabsf(fmaf(kS32, xb[e], 0.5f * xa[e]))));
+        }
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            if (!act[s] || i >= ng8) continue;
+            const uint4 t = reinterpret_cast<const uint4*>(p.Vt[s >> 1] + (size_t)(s & 1) * p.cols)[i];
+            const uint32_t t4[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                sv[s] = fmaf(xa[e], h2f((uint16_t)(t4[e] & 0xFFFFu)), sv[s]);
+                sv[s] = fmaf(xb[e], h2f((uint16_t)(t4[e] >> 16)), sv[s]);
+            }
+        }
+    }
+    {
+        const float t = wave_max_nonneg(mx);
+        if (lane == 0) red[wid][NS] = t;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        if (!act[s]) continue;
+        const float t = wave_sum_valu(sv[s]);
+        if (lane == 0) red[wid][s] = t;
+    }
+    __syncthreads();
+    mx = red[0][NS];
+#pragma unroll
+    for (int q = 1; q < 8; q++) mx = fmaxf(mx, red[q][NS]);
+    if (valid && tid < NS && (tid & 1) < p.k[tid >> 1]) {
+        float t = 0.f;
+        for (int q = 0; q < 8; q++) t += red[q][tid];
+        p.tmp[tid >> 1][(size_t)m * p.k[tid >> 1] + (tid & 1)] = t * p.S[tid >> 1][tid & 1];
+    }
+    int ex = 0;
+    if (mx > 0.f && mx < INFINITY) (void)frexpf(mx, &ex);
+    const float up = ldexpf(1.f, 14 - ex);
+    if (tid == 0) p.xs[m] = valid ? ldexpf(1.f, ex - 14) : 0.f;
+    const int g16 = m >> 4, ml = m & 15;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = tid + 512 * k;   // pairs 4 i .. 4 i + 3 (zeros past the row: chunk padding)
+        if (i >= nc * 16) continue;
+        const int q0 = 4 * i, c = q0 >> 6, h = (q0 >> 5) & 1, lg = (q0 >> 3) & 3, t2 = (q0 >> 2) & 1;
+        const uint32_t w4[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        uint32_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float xa = __uint_as_float(w4[e] << 16), xb = __uint_as_float(w4[e] & 0xFFFF0000u);
+            const float u = xa * up, vv = fmaf(kS32, xb, 0.5f * xa) * up;
+            o[e] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)u) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)vv) << 16);
+        }
+        p.xa[(((size_t)g16 * nc + c) * 4 + h * 2 + t2) * 64 + ml + 16 * lg] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 template <int TB, bool HL, int R2, int T2>
 hipError_t launch_hexmm32_t(const MmArgs& a, int grid, hipStream_t st) {
     const int lds = kMmStages * 2 * T2 * (HL ? 4 : 2) * 1024 + TB * 128;
@@ -578,6 +676,24 @@ MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols) {
     MmTile t{ng <= 4 ? 1 : 2, ng <= 2 ? 1 : 2, 1};
     const int rb = 8 * t.r2, tiles = ((rows_total_tiles_of_16 + rb - 1) / rb) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
     t.nsplit = whole_splits(nc, std::max(1, std::min({2 * ncu / tiles, nc / 4, 16})));
+    return t;
+}
+
+// Single operands (gsdh_model_matmul), one tensor of a call (tensors of one
+// call tile alike, so a launch may hold several): one row tile per wave and 32, 64 or
+// 128 tokens.  nsplit 0: hexmm_kernel, where the columns would have to be
+// split and the partial sums' passes (8 bytes per split and output) come to
+// more than about the decode of the weights they spare: measured at 512
+// tokens 4096 x 4096, 37 us there against 31 + 13 here; 4096 x 14336 in four
+// splits 110 against 75 + 13; 28672 x 4096 at 128 tokens in two 57 against
+// 48 + 8, 6144 x 4096 at 16 tokens 13 + 4 (three launches of each) against 9 + 3.
+MmTile hexmm32_tile(int M, int rows, int cols) {
+    const int ng = (M + 15) / 16, nc = (cols + 127) / 128, ncu = device_cu_count() > 0 ? device_cu_count() : 256;
+    MmTile t{1, ng <= 2 ? 1 : (ng <= 4 ? 2 : 4), 0};
+    const int tiles = ((rows + 127) / 128) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
+    const int s = whole_splits(nc, std::max(1, std::min({(nc >= 64 ? 2 * ncu : ncu) / tiles, nc / 4, 16})));
+    const bool ok = ng <= 4 || (s == 1 ? 4 * tiles >= 3 * ncu : 32LL * s * ng * 16 <= 5LL * cols);
+    t.nsplit = ok && rows % 4 == 0 ? s : 0;
     return t;
 }
 
@@ -626,6 +742,19 @@ hipError_t launch_mm_reduce(const MmArgs& a, hipStream_t st) {
     }
     if (!n) return hipSuccess;
     hipLaunchKernelGGL(mm_reduce_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096), a.nseg), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+bool mm_xprep_covers(const MmXprep& p) {
+    if (p.cols > 16384 || (reinterpret_cast<uintptr_t>(p.X) & 15)) return false;
+    for (int s = 0; s < kMaxSeg; s++)
+        if (p.k[s] > 2 || (p.k[s] > 0 && (reinterpret_cast<uintptr_t>(p.Vt[s]) & 15))) return false;
+    return true;
+}
+
+hipError_t launch_mm_xprep(const MmXprep& p, hipStream_t st) {
+    if (p.M <= 0 || p.cols <= 0 || p.cols % 64 || !p.X || !p.xa || !p.xs || !mm_xprep_covers(p)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(mm_xprep_kernel, dim3(((p.M + 15) / 16) * 16), dim3(512), 0, st, p);
     return hipGetLastError();
 }
 
