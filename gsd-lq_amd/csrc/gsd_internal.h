@@ -469,6 +469,8 @@ struct PrefillAttn {
     int log2g;   // set by the launcher
 };
 hipError_t launch_prefill_attention(const PrefillAttn& a, hipStream_t stream);
+// its kernel for head dims 64 and 128 (gsd_prefill.hip; log2g set)
+hipError_t launch_attn_prompt(const PrefillAttn& a, dim3 grid, hipStream_t stream);
 // RoPE + K/V append at a.pos fused into the one-token attention launch
 // (host position; k, v: the new rows before RoPE; cs: (cos, sin) of pos,
 // hd / 2 pairs): q is rotated in place, the cache rows written, out as

@@ -3341,8 +3341,8 @@ __global__ void __launch_bounds__(256) hexmm_reduce_kernel(const MatmulArgs a) {
 }
 
 // ------------------------------------------------------------------------
-// Causal attention of a batch of prompt tokens on the matrix cores.  Each
-// token computes what the reference's one-token attention computes
+// Causal attention of a batch of prompt tokens on the matrix cores, head dim
+// 256 (attn_prompt_kernel's registers do not hold its output).  Each token computes what the reference's one-token attention computes
 // (gsd_lq_cpu_engine.c:264-330; the reference prefills token by token,
 // run_gpu_native_chat.py:1128-1130): token t of the batch sits at position
 // p0 + t and attends over cache positions 0 .. p0 + t.
@@ -4123,8 +4123,8 @@ hipError_t launch_prefill_attention(const PrefillAttn& a, hipStream_t st) {
     const int T = 64 / G;
     const dim3 grid((a.M + T - 1) / T, a.n_kv);
     switch (a.hd) {
-        case 64: hipLaunchKernelGGL((attn_prefill_kernel<64>), grid, dim3(256), 0, st, b); break;
-        case 128: hipLaunchKernelGGL((attn_prefill_kernel<128>), grid, dim3(256), 0, st, b); break;
+        case 64:
+        case 128: return launch_attn_prompt(b, grid, st);
         case 256: hipLaunchKernelGGL((attn_prefill_kernel<256>), grid, dim3(256), 0, st, b); break;
         default: return hipErrorInvalidValue;
     }

@@ -634,6 +634,262 @@ __global__ void __launch_bounds__(512) mm_xprep_kernel(const MmXprep p) {
     }
 }
 
+// ------------------------------------------------------------------------
+// Causal attention of a batch of prompt tokens, head dims 64 and 128 (the
+// arithmetic of attn_prefill_kernel, which keeps 256): token t of the batch
+// at position p0 + t attends over cache positions 0 .. p0 + t.
+// Block: KV head blockIdx.y and 64 query rows (T = 64 / G tokens x the G
+// heads of the KV head), 8 waves: wave rt of a pair holds rows 32 rt .. + 31,
+// one per lane column, and the four pairs take the 32-position chunks of the
+// context in turn (c = pair, pair + 4, ..), each with LDS buffers of its own
+// and one barrier per four chunks; their (max, sum, output) are merged in LDS
+// at the end, in pair order.
+// Bound: a wave's serial chain scores -> softmax -> output.  A block per 64
+// rows fills 256 CUs with one wave per SIMD at 512 tokens, whose chain of 16 x
+// 16 products took 2.2 us per 32 positions (107 us for 512 tokens behind 1024,
+// 10 % of the matrix cores' rate; 32 us for 37 tokens behind 301, on 24 CUs).
+// Splitting the context over pairs puts two waves on every SIMD and cuts the
+// chain to a quarter; 32 x 32 products halve the LDS reads per row and leave
+// a row's positions in two lanes; scores are masked only in chunks that reach
+// past a row, and the output is rescaled only where a maximum moved.  Now 38
+// us for the 512 tokens (0.56 PFLOP/s of matrix-core work).
+// Scores: q as fp16 high + low parts after a per-row power of two (~22 bits),
+// probabilities as high + low parts; K and V exact.  Positions past the
+// block's last token are staged as zeros (cache rows there may hold anything).
+// ------------------------------------------------------------------------
+template <int HD>
+__global__ void __launch_bounds__(512, 2) attn_prompt_kernel(const PrefillAttn a) {
+    constexpr int NP = 4;         // pairs of waves
+    constexpr int KS = HD + 8;    // K row stride, halves (16 bytes of padding)
+    constexpr int VS = 36;        // V^T row stride, halves (32 positions + 4)
+    constexpr int NKS = HD / 16;  // steps of the scores
+    constexpr int NDT = HD / 32;  // 32-dimension tiles of the output
+    constexpr int D8 = HD / 8;    // 16-byte pieces of a cache row
+    constexpr int NK = 32 * D8 / 128, NV = 16 * D8 / 128;   // K pieces, V pairs of pieces per thread and chunk
+    constexpr uint32_t KB = 32 * KS * 2, BUF = KB + HD * VS * 2;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_pa[];   // [pair][2][K rows | V^T rows], then the merge
+    const int tid = threadIdx.x, lane = tid & 63, gt = tid & 127;
+    const int pair = __builtin_amdgcn_readfirstlane(tid >> 7), rt = __builtin_amdgcn_readfirstlane((tid >> 6) & 1);
+    const int n = lane & 31, kg = lane >> 5;
+    const int lg = a.log2g, G = 1 << lg, T = 64 >> lg;
+    const int grp = (int)gridDim.x - 1 - (int)blockIdx.x;   // the longest blocks first
+    const int kvh = (int)blockIdx.y, t0 = grp * T;
+    const int r = 32 * rt + n;
+    const int t = t0 + (r >> lg), head = kvh * G + (r & (G - 1));
+    const bool valid = t < a.M;
+    const int limit = a.p0 + t;   // last position of this row
+    const int maxpos = a.p0 + min(t0 + T, a.M) - 1;
+    const int nch = maxpos / 32 + 1, nround = (nch + NP - 1) / NP;
+    const int full = (a.p0 + t0 + ((32 * rt) >> lg) + 1) / 32;   // chunks below every row of this wave
+
+    half8v qh[NKS], ql[NKS];   // B: row n, dims 16 ks + 8 kg ..
+    float down;
+    {
+        const float qs = a.sm_scale * 1.44269504088896340736f;
+        const float* qr = a.q + ((size_t)(valid ? t : 0) * a.n_heads + head) * HD + 8 * kg;
+        float qv[NKS][8];
+        float mx = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ks++) {
+            float4 f0 = make_float4(0.f, 0.f, 0.f, 0.f), f1 = f0;
+            if (valid) {
+                f0 = *reinterpret_cast<const float4*>(qr + 16 * ks);
+                f1 = *reinterpret_cast<const float4*>(qr + 16 * ks + 4);
+            }
+            const float v8[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                qv[ks][j] = v8[j] * qs;
+                mx = fmaxf(mx, fabsf(qv[ks][j]));
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        int ex = 0;
+        if (mx > 0.f && mx < INFINITY) (void)frexpf(mx, &ex);
+        const float up = ldexpf(1.f, 14 - ex);
+        down = ldexpf(1.f, ex - 14);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ks++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float x = qv[ks][j] * up;
+                const _Float16 h = (_Float16)x;
+                qh[ks][j] = h;
+                ql[ks][j] = (_Float16)(x - (float)h);
+            }
+    }
+
+    const size_t rstride = (size_t)a.n_kv * HD;   // halves from one position to the next
+    const size_t lbase = ((size_t)a.layer * a.max_seq * a.n_kv + kvh) * HD;
+    const uint16_t* kbase = a.k_cache + lbase;
+    const uint16_t* vbase = a.v_cache + lbase;
+    u32x4v kr[NK], vr[NV][2];
+    const u32x4v z4 = {0u, 0u, 0u, 0u};
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NK; i++) {
+            const int idx = gt + 128 * i, p = 32 * c + idx / D8;
+            kr[i] = p <= maxpos ? *reinterpret_cast<const u32x4v*>(kbase + (size_t)p * rstride + (idx % D8) * 8) : z4;
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {   // pairs of positions (low bits) x pieces
+            const int idx = gt + 128 * i, p = 32 * c + 2 * (idx & 15);
+            const size_t off = (size_t)p * rstride + (idx >> 4) * 8;
+            vr[i][0] = p <= maxpos ? *reinterpret_cast<const u32x4v*>(vbase + off) : z4;
+            vr[i][1] = p + 1 <= maxpos ? *reinterpret_cast<const u32x4v*>(vbase + off + rstride) : z4;
+        }
+    };
+    unsigned char* const mine = lds_pa + (uint32_t)pair * 2u * BUF;
+    auto put = [&](int b) {
+        uint16_t* kl = reinterpret_cast<uint16_t*>(mine + b * BUF);
+        uint32_t* vw = reinterpret_cast<uint32_t*>(mine + b * BUF + KB);
+#pragma unroll
+        for (int i = 0; i < NK; i++) {
+            const int idx = gt + 128 * i;
+            *reinterpret_cast<u32x4v*>(kl + (idx / D8) * KS + (idx % D8) * 8) = kr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int idx = gt + 128 * i, j = idx & 15, d0 = (idx >> 4) * 8;
+#pragma unroll
+            for (int e = 0; e < 8; e++)   // dim d0 + e of positions 2 j, 2 j + 1
+                vw[(d0 + e) * (VS / 2) + j] = __builtin_amdgcn_perm(vr[i][1][e >> 1], vr[i][0][e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+        }
+    };
+
+    float16v o[NDT];
+#pragma unroll
+    for (int d = 0; d < NDT; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[d][i] = 0.f;
+    float mrun = -INFINITY, lsum = 0.f;
+    if (pair < nch) {
+        fetch(pair);
+        put(0);
+    }
+    __syncthreads();
+    for (int i = 0; i < nround; i++) {
+        const int c = pair + NP * i;
+        if (c + NP < nch) fetch(c + NP);
+        if (c < nch) {
+            const uint16_t* kb = reinterpret_cast<const uint16_t*>(mine + (i & 1) * BUF);
+            const uint16_t* vb = reinterpret_cast<const uint16_t*>(mine + (i & 1) * BUF + KB);
+            float16v sh, sl;
+#pragma unroll
+            for (int j = 0; j < 16; j++) sh[j] = sl[j] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ks++) {
+                const half8v ka = *reinterpret_cast<const half8v*>(kb + n * KS + 16 * ks + 8 * kg);
+                sh = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[ks], sh, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[ks], sl, 0, 0, 0);
+            }
+            // lane: row n, positions 32 c + 8 (j >> 2) + 4 kg + (j & 3)
+            float s[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) s[j] = (sh[j] + sl[j]) * down;
+            if (c >= full) {
+#pragma unroll
+                for (int j = 0; j < 16; j++)
+                    if (32 * c + 8 * (j >> 2) + 4 * kg + (j & 3) > limit) s[j] = -INFINITY;
+            }
+            float mc = s[0];
+#pragma unroll
+            for (int j = 1; j < 16; j++) mc = fmaxf(mc, s[j]);
+            mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
+            const float mnew = fmaxf(mrun, mc);
+            const float base = mnew == -INFINITY ? 0.f : mnew;   // (a chunk past this row: all masked)
+            if (__any(mnew != mrun)) {
+                const float alpha = __builtin_amdgcn_exp2f(mrun - base);
+                lsum *= alpha;
+#pragma unroll
+                for (int d = 0; d < NDT; d++)
+#pragma unroll
+                    for (int j = 0; j < 16; j++) o[d][j] *= alpha;
+                mrun = mnew;
+            }
+            half8v ph[2], pl[2];
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const float pj = __builtin_amdgcn_exp2f(s[j] - base);
+                lsum += pj;
+                const _Float16 h = (_Float16)pj;
+                ph[j >> 3][j & 7] = h;
+                pl[j >> 3][j & 7] = (_Float16)(pj - (float)h);
+            }
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+#pragma unroll
+                for (int d = 0; d < NDT; d++) {   // A: dim 32 d + n, positions 16 st + 4 kg .. + 3 and 8 on
+                    const uint16_t* vrow = vb + (32 * d + n) * VS + 16 * st + 4 * kg;
+                    const uint2 lo4 = *reinterpret_cast<const uint2*>(vrow), hi4 = *reinterpret_cast<const uint2*>(vrow + 8);
+                    const u32x4v vw = {lo4.x, lo4.y, hi4.x, hi4.y};
+                    const half8v va = __builtin_bit_cast(half8v, vw);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph[st], o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl[st], o[d], 0, 0, 0);
+                }
+            }
+        }
+        if (c + NP < nch) put((i + 1) & 1);
+        __syncthreads();
+    }
+    lsum += __shfl_xor(lsum, 32, 64);
+
+    // merge the pairs: maxima and sums, then the scaled outputs, dim tile d
+    // of a row tile summed and stored by its pair d
+    float2* ml = reinterpret_cast<float2*>(lds_pa);          // [rt][pair][32 rows]
+    float4* ob = reinterpret_cast<float4*>(lds_pa + 2048);   // [rt][pair][tile][4][64 lanes]
+    if (kg == 0) ml[(rt * NP + pair) * 32 + n] = make_float2(mrun, lsum);
+    __syncthreads();
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; p++) M = fmaxf(M, ml[(rt * NP + p) * 32 + n].x);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const float2 v = ml[(rt * NP + p) * 32 + n];
+        L += v.y * __builtin_amdgcn_exp2f(v.x - M);
+    }
+    const float f = __builtin_amdgcn_exp2f(mrun - M);
+#pragma unroll
+    for (int d = 0; d < NDT; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            ob[(((rt * NP + pair) * NDT + d) * 4 + j) * 64 + lane] =
+                make_float4(o[d][4 * j] * f, o[d][4 * j + 1] * f, o[d][4 * j + 2] * f, o[d][4 * j + 3] * f);
+    __syncthreads();
+    if (pair < NDT && valid) {
+        const float inv = 1.0f / L;
+        float* out = a.out + ((size_t)t * a.n_heads + head) * HD + 32 * pair + 4 * kg;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const float4 v = ob[(((rt * NP + p) * NDT + pair) * 4 + j) * 64 + lane];
+                y.x += v.x;
+                y.y += v.y;
+                y.z += v.z;
+                y.w += v.w;
+            }
+            *reinterpret_cast<float4*>(out + 8 * j) = make_float4(y.x * inv, y.y * inv, y.z * inv, y.w * inv);
+        }
+    }
+}
+
+template <int HD>
+hipError_t launch_attn_prompt_t(const PrefillAttn& a, dim3 grid, hipStream_t st) {
+    constexpr int lds = 4 * 2 * (32 * (HD + 8) * 2 + HD * 36 * 2);
+    static_assert(lds >= 2048 + 2 * 4 * (HD / 32) * 4 * 64 * 16 && lds <= 160 * 1024, "the merge fits the stages");
+    static bool attr = false;
+    if (!attr) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prompt_kernel<HD>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    hipLaunchKernelGGL((attn_prompt_kernel<HD>), grid, dim3(512), lds, st, a);
+    return hipGetLastError();
+}
+
 template <int TB, bool HL, int R2, int T2>
 hipError_t launch_hexmm32_t(const MmArgs& a, int grid, hipStream_t st) {
     const int lds = kMmStages * 2 * T2 * (HL ? 4 : 2) * 1024 + TB * 128;
@@ -663,6 +919,12 @@ hipError_t launch_hexmm32_tb(const MmArgs& a, int grid, hipStream_t st) {
 }
 
 }  // namespace
+
+hipError_t launch_attn_prompt(const PrefillAttn& a, dim3 grid, hipStream_t st) {
+    if (a.hd == 64) return launch_attn_prompt_t<64>(a, grid, st);
+    if (a.hd == 128) return launch_attn_prompt_t<128>(a, grid, st);
+    return hipErrorInvalidValue;
+}
 
 bool hexmm32_codebook(int n_pts) { return n_pts == 217 || n_pts == 127; }
 

@@ -56,6 +56,17 @@ def test_matmul_edges(mode, kpr, shape, M):
         model.close()
 
 
+# 32-position chunks taken in turn by four pairs of waves: contexts of fewer
+# chunks than pairs, one position past and short of a chunk, of a round of
+# chunks; 64 query rows of 8, 16, 32 and 64 tokens, and one token more
+@pytest.mark.parametrize("p0,M", [(0, 2), (31, 2), (0, 33), (95, 34), (127, 3), (128, 65), (3, 130), (255, 9)])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 1, 128), (4, 4, 64), (4, 2, 128), (16, 4, 64)])
+def test_prompt_attention_edges(p0, M, nh, nkv, hd):
+    import test_gpu_ops
+    from gsdlq import hip
+    test_gpu_ops.test_prefill_attention_vs_oracle(hip.lib(), p0, M, nh, nkv, hd, 1, p0 + M + 3)
+
+
 @pytest.mark.parametrize("mode,shape", [("precision", dict()), ("precision", dict(k_dim=3))])
 def test_any_number_of_prompts(mode, shape):
     """Each prompt's head took further publication words of the model until,
