@@ -513,7 +513,11 @@ struct gsdh_model {
     bool offn_on = true;                 // the o projection in the same launch (GSD_FUSED_OFFN=0: off)
     int chunk = 64, max_splits = 1;
     StepState* st = nullptr;        // device
-    StepState* st_host = nullptr;   // pinned
+    // pinned: [0] a step's token and position, [1] the finished step state; the
+    // head's logits; token ids of a prompt (max_seq_len)
+    StepState* st_host = nullptr;
+    float* logits_host = nullptr;
+    int* tok_host = nullptr;
     int* gen_tok = nullptr;
     float* gen_margin = nullptr;
     // per-token graphs: with and without the lm_head / argmax, for any
@@ -522,6 +526,9 @@ struct gsdh_model {
     // loads the chunk's rows before it reads the position)
     hipGraphExec_t g_full = nullptr, g_prefill = nullptr;
     hipGraphExec_t g_full_s[kShortTiers] = {}, g_prefill_s[kShortTiers] = {};
+    // the same with the head for forward_token: the token and position come
+    // from st_host[0], the logits and the finished state go to the pinned buffers
+    hipGraphExec_t g_step = nullptr, g_step_s[kShortTiers] = {};
     hipGraph_t capture_graph = nullptr;
     size_t dev_bytes = 0;
     bool finalized = false;
@@ -712,8 +719,9 @@ int issue_linear(gsdh_model* m, int l, int mask) {
 }
 
 // Final RMSNorm + lm_head (run_gpu_native_chat.py:962-968) and, with
-// `greedy`, the device argmax that appends the token and advances the step.
-int issue_head(gsdh_model* m, bool greedy) {
+// `greedy`, the device argmax that appends the token and advances the step
+// (to_host: and leaves the logits and the state in the pinned buffers).
+int issue_head(gsdh_model* m, bool greedy, bool to_host = false) {
     const auto& c = m->c;
     HexArgs a{};
     a.nseg = 1;
@@ -724,7 +732,8 @@ int issue_head(gsdh_model* m, bool greedy) {
     if (rc) return rc;
     HIPCHK(launch_hexmv4(a, m->stream));
     if (greedy)
-        HIPCHK(launch_argmax(m->logits, c.vocab, m->st, m->gen_tok, m->gen_margin, 1, m->stream, m->am_words, m->am_ctr));
+        HIPCHK(launch_argmax(m->logits, c.vocab, m->st, m->gen_tok, m->gen_margin, 1, m->stream, m->am_words, m->am_ctr,
+                             to_host ? m->logits_host : nullptr, to_host ? m->st_host + 1 : nullptr));
     return 0;
 }
 
@@ -747,11 +756,12 @@ AttnArgs layer_attention(gsdh_model* m, int l, int short_chunk) {
 
 // The per-token launch sequence (run_gpu_native_chat.py:892-969, fused).
 // short_chunk: 0 for the graph of any position, else the single attention
-// chunk (64, 128 or 256) of the graph for positions below it
-int issue_token(gsdh_model* m, bool with_head, int short_chunk) {
+// chunk (64, 128 or 256) of the graph for positions below it; host: token and
+// position from the pinned step, results to the pinned buffers
+int issue_token(gsdh_model* m, bool with_head, int short_chunk, bool host) {
     const auto& c = m->c;
     m->pub_next = 0;
-    HIPCHK(launch_embed(m->embed, &m->st->token, m->x, c.hidden, m->pub, m->pub_words, m->fa_epoch, m->stream));
+    HIPCHK(launch_embed(m->embed, m->st, host ? m->st_host : nullptr, m->x, c.hidden, m->pub, m->pub_words, m->fa_epoch, m->stream));
     for (int l = 0; l < c.n_layers; l++) {
         // positions < 256: the attention in the q/k/v launch where it covers the model
         bool fused = false;
@@ -775,7 +785,7 @@ int issue_token(gsdh_model* m, bool with_head, int short_chunk) {
         rc = issue_linear(m, l, 2 | 4 | 8);
         if (rc) return rc;
     }
-    if (with_head) return issue_head(m, true);
+    if (with_head) return issue_head(m, true, host);
     return 0;
 }
 
@@ -783,6 +793,11 @@ hipGraphExec_t token_graph(const gsdh_model* m, bool with_head, int pos) {
     for (int t = 0; t < kShortTiers; t++)
         if (pos < kShortChunk[t]) return with_head ? m->g_full_s[t] : m->g_prefill_s[t];
     return with_head ? m->g_full : m->g_prefill;
+}
+hipGraphExec_t step_graph(const gsdh_model* m, int pos) {
+    for (int t = 0; t < kShortTiers; t++)
+        if (pos < kShortChunk[t]) return m->g_step_s[t];
+    return m->g_step;
 }
 
 // Staging bytes of one gsdh_model_matmul call (bf16 X, single fp16 operand
@@ -1102,18 +1117,19 @@ int issue_prompt32(gsdh_model* m, int M, int p0, bool last) {
 // Prompt prompt[0..n) at positions start.. in batches of the prefill chunk;
 // with `head`, the last token's logits and the greedy step (the step state
 // then holds the first generated token at position start + n, gen_count 1).
-// tok_stage: pinned host staging of n token ids (read by the copies until
-// the stream is synchronised).  The step state's error word is cleared
+// The token ids go through the pinned tok_host (read by the copies until the
+// stream is synchronised); to_host: the logits and the finished state are
+// left in the pinned buffers.  The step state's error word is cleared
 // first and then only ever set, so a bounded wait that ran out in any
 // chunk's attention reaches the caller.
-int run_prefill(gsdh_model* m, const int* prompt, int n, int start, bool head, int* tok_stage) {
+int run_prefill(gsdh_model* m, const int* prompt, int n, int start, bool head, bool to_host) {
     auto& P = m->pf;
     // the step state of the last token from the start: the 32 x 32 tile path
     // runs that token's last layer as a decode step
     HIPCHK(launch_set_step(m->st, prompt[n - 1], start + n - 1, 1, m->stream));
     for (int b0 = 0; b0 < n; b0 += P.chunk) {
         const int M = std::min(P.chunk, n - b0);
-        int* ts = tok_stage + b0;
+        int* ts = m->tok_host + b0;
         for (int i = 0; i < M; i++) ts[i] = prompt[b0 + i];
         HIPCHK(hipMemcpyAsync(P.tok, ts, (size_t)M * 4, hipMemcpyHostToDevice, m->stream));
         int rc = P.xs1 ? issue_prompt32(m, M, start + b0, b0 + M == n) : issue_prefill(m, M, start + b0);
@@ -1124,13 +1140,13 @@ int run_prefill(gsdh_model* m, const int* prompt, int n, int start, bool head, i
     // on, cleared: each prompt took the next ones until none were left
     m->pub_next = 0;
     if (m->slot(0, GSDH_LM_HEAD).k > 2) HIPCHK(launch_fill_u32((unsigned*)m->pub, 0u, 2 * (size_t)kLeadMax, m->stream));
-    return issue_head(m, true);
+    return issue_head(m, true, to_host);
 }
 
-int capture(gsdh_model* m, bool with_head, int short_chunk, hipGraphExec_t* out) {
+int capture(gsdh_model* m, bool with_head, int short_chunk, hipGraphExec_t* out, bool host = false) {
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-    int rc = issue_token(m, with_head, short_chunk);
+    int rc = issue_token(m, with_head, short_chunk, host);
     hipError_t e = hipStreamEndCapture(m->stream, &g);
     if (rc) {
         if (g) (void)hipGraphDestroy(g);
@@ -1222,6 +1238,8 @@ int gsdh_model_create(const gsdh_model_config* cfg, gsdh_model** out) {
     }
     if (!rc) {
         e = hipHostMalloc((void**)&m->st_host, sizeof(StepState) * 2, 0);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&m->logits_host, (size_t)c.vocab * 4, 0);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&m->tok_host, (size_t)c.max_seq_len * 4, 0);
         if (e != hipSuccess) rc = fail((int)e, "hipHostMalloc: %s", hipGetErrorString(e));
     }
     if (!rc) {
@@ -1262,15 +1280,16 @@ int gsdh_model_create(const gsdh_model_config* cfg, gsdh_model** out) {
 int gsdh_model_destroy(gsdh_model* m) {
     if (!m) return 0;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    for (hipGraphExec_t g : {m->g_full, m->g_prefill})
+    for (hipGraphExec_t g : {m->g_full, m->g_prefill, m->g_step})
         if (g) (void)hipGraphExecDestroy(g);
     for (int t = 0; t < kShortTiers; t++)
-        for (hipGraphExec_t g : {m->g_full_s[t], m->g_prefill_s[t]})
+        for (hipGraphExec_t g : {m->g_full_s[t], m->g_prefill_s[t], m->g_step_s[t]})
             if (g) (void)hipGraphExecDestroy(g);
     for (auto& t : m->hex)
         if (t.block) (void)hipFree(t.block);
     for (void* p : m->allocs) (void)hipFree(p);
-    if (m->st_host) (void)hipHostFree(m->st_host);
+    for (void* p : {(void*)m->st_host, (void*)m->logits_host, (void*)m->tok_host})
+        if (p) (void)hipHostFree(p);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
     return 0;
@@ -1443,9 +1462,11 @@ int gsdh_model_finalize(gsdh_model* m) {
     if (!m->slot(0, GSDH_LM_HEAD).set) return fail(-1, "finalize: lm_head not set");
     int rc = capture(m, true, 0, &m->g_full);
     if (!rc) rc = capture(m, false, 0, &m->g_prefill);
+    if (!rc) rc = capture(m, true, 0, &m->g_step, true);
     for (int t = 0; t < kShortTiers && !rc; t++) {
         rc = capture(m, true, kShortChunk[t], &m->g_full_s[t]);
         if (!rc) rc = capture(m, false, kShortChunk[t], &m->g_prefill_s[t]);
+        if (!rc) rc = capture(m, true, kShortChunk[t], &m->g_step_s[t], true);
     }
     if (!rc) rc = setup_batched(m);
     if (rc) return rc;
@@ -1463,13 +1484,16 @@ int gsdh_forward_token(gsdh_model* m, int token_id, int pos, int want_logits, fl
     StepState* h = m->st_host;
     *h = StepState{};
     h->token = token_id; h->pos = pos;
-    HIPCHK(hipMemcpyAsync(m->st, h, sizeof(StepState), hipMemcpyHostToDevice, m->stream));
-    HIPCHK(hipGraphLaunch(token_graph(m, want_logits != 0, pos), m->stream));
-    if (want_logits && logits_host)
-        HIPCHK(hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, m->stream));
-    HIPCHK(hipMemcpyAsync(m->st_host + 1, m->st, sizeof(StepState), hipMemcpyDeviceToHost, m->stream));
+    if (want_logits) {   // one launch: the graph reads the step and leaves its results in pinned memory
+        HIPCHK(hipGraphLaunch(step_graph(m, pos), m->stream));
+    } else {
+        HIPCHK(hipMemcpyAsync(m->st, h, sizeof(StepState), hipMemcpyHostToDevice, m->stream));
+        HIPCHK(hipGraphLaunch(token_graph(m, false, pos), m->stream));
+        HIPCHK(hipMemcpyAsync(m->st_host + 1, m->st, sizeof(StepState), hipMemcpyDeviceToHost, m->stream));
+    }
     HIPCHK(hipStreamSynchronize(m->stream));
     if (m->st_host[1].err) return fail(-2, "forward_token: an in-kernel wait timed out");
+    if (want_logits && logits_host) std::memcpy(logits_host, m->logits_host, (size_t)m->c.vocab * 4);
     if (want_logits && argmax_out) *argmax_out = m->st_host[1].token;
     return 0;
 }
@@ -1482,11 +1506,9 @@ int gsdh_generate_greedy(gsdh_model* m, const int* prompt, int n_prompt, int sta
         return fail(-1, "generate: positions %d..%d exceed max_seq_len %d", start_pos, start_pos + n_prompt + n_new - 1, m->c.max_seq_len);
     for (int i = 0; i < n_prompt; i++)
         if (prompt[i] < 0 || prompt[i] >= m->c.vocab) return fail(-1, "generate: prompt token %d outside vocab", prompt[i]);
-    int* tok_stage = nullptr;
-    HIPCHK(hipHostMalloc((void**)&tok_stage, sizeof(int) * (size_t)n_prompt, 0));
     int rc = 0;
     if (m->pf.batched) {
-        rc = run_prefill(m, prompt, n_prompt, start_pos, true, tok_stage);
+        rc = run_prefill(m, prompt, n_prompt, start_pos, true, false);
     } else {
         // token by token: the step state of each prompt token, its error
         // word cleared for the first only (a wait that ran out stays set)
@@ -1511,7 +1533,6 @@ int gsdh_generate_greedy(gsdh_model* m, const int* prompt, int n_prompt, int sta
         else if (m->st_host[1].err) rc = fail(-2, "generate: an in-kernel wait timed out");
     }
     (void)hipStreamSynchronize(m->stream);
-    (void)hipHostFree(tok_stage);
     return rc;
 }
 
@@ -1524,23 +1545,18 @@ int gsdh_model_prefill(gsdh_model* m, const int* tokens, int n, int start_pos, i
         return fail(-1, "prefill: positions %d..%d exceed max_seq_len %d", start_pos, start_pos + n - 1, m->c.max_seq_len);
     for (int i = 0; i < n; i++)
         if (tokens[i] < 0 || tokens[i] >= m->c.vocab) return fail(-1, "prefill: token %d outside vocab %d", tokens[i], m->c.vocab);
-    StepState* ring = nullptr;
-    HIPCHK(hipHostMalloc((void**)&ring, sizeof(StepState) * 2 + sizeof(int) * (size_t)n, 0));
-    int rc = run_prefill(m, tokens, n, start_pos, want_logits != 0, reinterpret_cast<int*>(ring + 2));
-    if (!rc && want_logits && logits_host) {
-        hipError_t e = hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, m->stream);
+    int rc = run_prefill(m, tokens, n, start_pos, want_logits != 0, want_logits != 0);
+    if (!rc && !want_logits) {
+        hipError_t e = hipMemcpyAsync(m->st_host + 1, m->st, sizeof(StepState), hipMemcpyDeviceToHost, m->stream);
         if (e != hipSuccess) rc = fail((int)e, "prefill: %s", hipGetErrorString(e));
     }
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(ring + 1, m->st, sizeof(StepState), hipMemcpyDeviceToHost, m->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-        if (e != hipSuccess) rc = fail((int)e, "prefill: %s", hipGetErrorString(e));
-        else if (ring[1].err) rc = fail(-2, "prefill: an in-kernel wait timed out");
-        else if (want_logits && argmax_out) *argmax_out = ring[1].token;
-    }
-    (void)hipStreamSynchronize(m->stream);
-    (void)hipHostFree(ring);
-    return rc;
+    hipError_t e = hipStreamSynchronize(m->stream);
+    if (rc) return rc;
+    if (e != hipSuccess) return fail((int)e, "prefill: %s", hipGetErrorString(e));
+    if (m->st_host[1].err) return fail(-2, "prefill: an in-kernel wait timed out");
+    if (want_logits && logits_host) std::memcpy(logits_host, m->logits_host, (size_t)m->c.vocab * 4);
+    if (want_logits && argmax_out) *argmax_out = m->st_host[1].token;
+    return 0;
 }
 
 int gsdh_model_fused_ffn(gsdh_model* m, int layer) {

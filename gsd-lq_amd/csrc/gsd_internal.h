@@ -525,17 +525,6 @@ int attention_static_error(int* was_set);
 // GSD_ATTN_SPIN_LIMIT -> spin_limit); both unset in use.
 void attention_test_knobs(AttnArgs& a);
 
-// embedding row of *token_dev to fp32 x; also zeroes clear[0..nclear) (the
-// rank-k publication words of the token's matvec launches) and, when epoch
-// is non-null, advances the token counter *epoch by one
-hipError_t launch_embed(const uint16_t* embed, const int* token_dev, float* x, int hidden,
-                        unsigned long long* clear, int nclear, unsigned* epoch, hipStream_t stream);
-
-// Greedy argmax with the reference's nan_to_num (gsd_lq_cpu_runtime.py:423);
-// with a step state st it writes the token and the margin top1-top2 there
-// and, when gen_tokens != null, appends both to the gen arrays at
-// st->gen_count (advance: st->pos += 1); with st == null it writes them to
-// gen_tokens[0] and gen_margins[0] only.
 struct StepState {
     int token;
     int pos;
@@ -544,12 +533,28 @@ struct StepState {
     unsigned err;       // nonzero: a bounded in-kernel wait timed out
     int pad[3];
 };
+// embedding row of the step's token to fp32 x; also zeroes clear[0..nclear)
+// (the rank-k publication words of the token's matvec launches) and, when
+// epoch is non-null, advances the token counter *epoch by one.  The token is
+// st->token or, with host_in (pinned host memory), host_in's token and
+// position, a fresh step state
+hipError_t launch_embed(const uint16_t* embed, StepState* st, const StepState* host_in, float* x, int hidden,
+                        unsigned long long* clear, int nclear, unsigned* epoch, hipStream_t stream);
+
+// Greedy argmax with the reference's nan_to_num (gsd_lq_cpu_runtime.py:423);
+// with a step state st it writes the token and the margin top1-top2 there
+// and, when gen_tokens != null, appends both to the gen arrays at
+// st->gen_count (advance: st->pos += 1); with st == null it writes them to
+// gen_tokens[0] and gen_margins[0] only.
 // words (3 kArgBlocks) and ctr (kArgBlocks, zero at first use, used by one
-// launch at a time): the multi-block form; otherwise one block
+// launch at a time): the multi-block form; otherwise one block.  host_logits,
+// host_st (multi-block with a step state only): pinned host memory that also
+// gets the logits and the finished step state
 constexpr int kArgBlocks = 32;
 hipError_t launch_argmax(const float* logits, int n, StepState* st, int* gen_tokens,
                          float* gen_margins, int advance, hipStream_t stream,
-                         unsigned long long* words = nullptr, unsigned* ctr = nullptr);
+                         unsigned long long* words = nullptr, unsigned* ctr = nullptr, float* host_logits = nullptr,
+                         StepState* host_st = nullptr);
 // st->token, pos = (token, pos), gen_count = 0; err cleared only with reset_err
 hipError_t launch_set_step(StepState* st, int token, int pos, int reset_err, hipStream_t stream);
 hipError_t launch_fill_u32(unsigned* p, unsigned v, size_t n, hipStream_t stream);

@@ -1469,10 +1469,23 @@ __global__ void set_step_kernel(StepState* st, int token, int pos, int reset_err
     if (reset_err) st->err = 0u;
 }
 
-__global__ void embed_kernel(const uint16_t* embed, const int* token, float* x, int hidden,
+// host_in (pinned host memory, or null): the step's token and position, which
+// the launch also puts into the step state; else the state's own token
+__global__ void embed_kernel(const uint16_t* embed, StepState* st, const StepState* host_in, float* x, int hidden,
                              unsigned long long* clear, int nclear, unsigned* epoch) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < hidden) x[i] = h2f(embed[(size_t)(*token) * hidden + i]);
+    int token;
+    if (host_in) {
+        token = __hip_atomic_load(&host_in->token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (i == 0) {
+            *st = StepState{};
+            st->token = token;
+            st->pos = __hip_atomic_load(&host_in->pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    } else {
+        token = st->token;
+    }
+    if (i < hidden) x[i] = h2f(embed[(size_t)token * hidden + i]);
     if (i < nclear) clear[i] = 0ull;
     if (i == 0 && epoch) *epoch += 1u;   // the token counter of the fused attention tags
 }
@@ -1548,7 +1561,10 @@ __global__ void __launch_bounds__(1024) argmax_kernel(const float* logits, int n
 // has started) polls the others' words (bounded: a wait that runs out sets
 // st->err), merges them and its own, and finishes as argmax_kernel.  Merging is order-free: the largest value
 // with the lowest index is a total order, the runner-up the second largest
-// of the union.
+// of the union.  host_logits / host_st (pinned host memory, or null): the
+// logits and the finished step state are written there too, by the blocks
+// that read them anyway, so a caller that wants them on the host waits for the stream
+// and needs no copy after it (2 copies and their waits: about 20 us of a call).
 __device__ __forceinline__ Top2 top2_add(Top2 t, float c, int i) {
     // i above every index seen: a tie keeps the earlier index
     const bool gt = c > t.v1;
@@ -1567,7 +1583,7 @@ __device__ __forceinline__ Top2 wave_top2(Top2 t) {
 }
 __global__ void __launch_bounds__(256) argmax_blocks_kernel(const float* logits, int n, StepState* st, int* gen_tok,
                                                             float* gen_margin, int advance, unsigned long long* words,
-                                                            unsigned* ctr) {
+                                                            unsigned* ctr, float* host_logits, StepState* host_st) {
     __shared__ Top2 sw[4];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int b = blockIdx.x, nb = gridDim.x;
@@ -1591,7 +1607,9 @@ __global__ void __launch_bounds__(256) argmax_blocks_kernel(const float* logits,
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int i = base + 256 * k;
-            if (i < e1) t = top2_add(t, clean(v[k]), i);
+            if (i >= e1) continue;
+            if (host_logits) host_logits[i] = v[k];
+            t = top2_add(t, clean(v[k]), i);
         }
     }
     t = wave_top2(t);
@@ -1633,6 +1651,7 @@ __global__ void __launch_bounds__(256) argmax_blocks_kernel(const float* logits,
         const Top2 r = merge(o, merge(merge(sw[0], sw[1]), merge(sw[2], sw[3])));
         ctr[b] = tag;
         argmax_finish(r, st, gen_tok, gen_margin, advance, c0, p0);
+        if (host_st) *host_st = *st;
     }
 }
 
@@ -4131,10 +4150,10 @@ hipError_t launch_prefill_attention(const PrefillAttn& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_embed(const uint16_t* embed, const int* token_dev, float* x, int hidden,
+hipError_t launch_embed(const uint16_t* embed, StepState* stt, const StepState* host_in, float* x, int hidden,
                         unsigned long long* clear, int nclear, unsigned* epoch, hipStream_t st) {
     const int n = hidden > nclear ? hidden : nclear;
-    hipLaunchKernelGGL(embed_kernel, dim3((n + 255) / 256), dim3(256), 0, st, embed, token_dev, x, hidden, clear,
+    hipLaunchKernelGGL(embed_kernel, dim3((n + 255) / 256), dim3(256), 0, st, embed, stt, host_in, x, hidden, clear,
                        nclear, epoch);
     return hipGetLastError();
 }
@@ -4145,10 +4164,12 @@ hipError_t launch_set_step(StepState* stt, int token, int pos, int reset_err, hi
 }
 
 hipError_t launch_argmax(const float* logits, int n, StepState* stt, int* gen_tokens, float* gen_margins,
-                         int advance, hipStream_t st, unsigned long long* words, unsigned* ctr) {
+                         int advance, hipStream_t st, unsigned long long* words, unsigned* ctr, float* host_logits,
+                         StepState* host_st) {
+    if ((host_logits || host_st) && !(words && ctr && stt)) return hipErrorInvalidValue;
     if (words && ctr)
         hipLaunchKernelGGL(argmax_blocks_kernel, dim3(kArgBlocks), dim3(256), 0, st, logits, n, stt, gen_tokens,
-                           gen_margins, advance, words, ctr);
+                           gen_margins, advance, words, ctr, host_logits, host_st);
     else
         hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, logits, n, stt, gen_tokens, gen_margins, advance);
     return hipGetLastError();

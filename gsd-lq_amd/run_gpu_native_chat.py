@@ -258,7 +258,6 @@ class GPUMistralV2Model:
         dev = int(lib.gsdh_model_device_bytes(self._m))
         self.cl.allocated_bytes = dev
         self.vram_used_mb = dev / (1024 * 1024)
-        self._logits = np.empty(self.vocab_size, dtype=np.float32)
 
     def _upload_hex(self, src, tensors, name, layer, slot):
         m = tensors[name]
@@ -300,9 +299,9 @@ class GPUMistralV2Model:
         logits (vocab,) when return_logits, else None (run_gpu_native_chat.py:892-969)."""
         am = ctypes.c_int(-1)
         if return_logits:
-            self.cl.lib.gsdh_forward_token(self._m, int(token_id), int(pos), 1, _hip.ptr(self._logits),
-                                           ctypes.byref(am))
-            return self._logits.copy()
+            logits = np.empty(self.vocab_size, dtype=np.float32)
+            self.cl.lib.gsdh_forward_token(self._m, int(token_id), int(pos), 1, _hip.ptr(logits), ctypes.byref(am))
+            return logits
         self.cl.lib.gsdh_forward_token(self._m, int(token_id), int(pos), 0, None, None)
         return None
 
@@ -318,9 +317,10 @@ class GPUMistralV2Model:
             raise ValueError("prefill: no tokens")
         am = ctypes.c_int(-1)
         if return_logits:
+            logits = np.empty(self.vocab_size, dtype=np.float32)
             self.cl.lib.gsdh_model_prefill(self._m, _hip.ptr(ids), int(ids.size), int(start_pos), 1,
-                                           _hip.ptr(self._logits), ctypes.byref(am))
-            return self._logits.copy()
+                                           _hip.ptr(logits), ctypes.byref(am))
+            return logits
         self.cl.lib.gsdh_model_prefill(self._m, _hip.ptr(ids), int(ids.size), int(start_pos), 0, None, None)
         return None
 
