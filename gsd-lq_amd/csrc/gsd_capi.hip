@@ -293,14 +293,11 @@ int gsdh_hex2d_matvec(void* stream, const float* x, const uint8_t* codes, const 
     if (k_dim < 0 || k_dim > kMaxRank) return fail(-1, "hex2d_matvec: k_dim %d outside 0..%d", k_dim, kMaxRank);
     if (n_pts <= 0 || n_pts > kTableSlots) return fail(-1, "hex2d_matvec: n_pts %d outside 1..256", n_pts);
     if (k_dim > 0 && (!U || !tmp_k)) return fail(-1, "hex2d_matvec: k_dim > 0 needs U and tmp_k");
-    HexArgs a{};
-    a.nseg = 1;
-    HexSeg& s = a.seg[0];
-    s.codes = codes; s.scales = scales; s.row_ptr = kink_row_ptr; s.kcols = kink_cols; s.kdel = kink_deltas;
-    s.U = U; s.Vt = nullptr; s.S = nullptr; s.tmp_k = tmp_k; s.table = xy_table; s.out = y;
-    s.rows = rows; s.k = k_dim; s.n_pts = n_pts;
-    a.x = x; a.norm_w = nullptr; a.eps = 0.f; a.resid = nullptr; a.cols = cols; a.epilogue = kEpiStore;
-    HIPCHK(launch_hexmv(a, S(stream)));
+    FileMatvec a{};
+    a.x = x; a.codes = codes; a.scales = scales; a.table = reinterpret_cast<const float2*>(xy_table); a.U = U; a.tmp_k = tmp_k;
+    a.row_ptr = kink_row_ptr; a.kcols = kink_cols; a.kdel = kink_deltas; a.y = y;
+    a.rows = rows; a.cols = cols; a.k = k_dim; a.n_pts = n_pts;
+    HIPCHK(launch_hexmv_file(a, S(stream)));
     return 0;
 }
 

@@ -203,7 +203,22 @@ constexpr int kFfnMaxGrid = 1024;
 bool ffn_supported(int hidden, int ffn);
 
 // Launches (all asynchronous on `stream`).
-hipError_t launch_hexmv(const HexArgs& a, hipStream_t stream);
+// y = W x (+ kinks, U tmp_k) over one packed tensor in the file's layout (the
+// operator twin; table: float2 [n_pts])
+struct FileMatvec {
+    const float* x;
+    const uint8_t* codes;
+    const uint16_t* scales;
+    const float2* table;
+    const uint16_t* U;         // k > 0
+    const float* tmp_k;
+    const uint32_t* row_ptr;   // null: no kinks
+    const uint16_t* kcols;
+    const float* kdel;
+    float* y;
+    int rows, cols, k, n_pts;
+};
+hipError_t launch_hexmv_file(const FileMatvec& a, hipStream_t stream);
 // MFMA matvec over the tiled layout (codes_t / scales_t / fields of every
 // segment); same epilogues, norm and rank-k handling as launch_hexmv.
 hipError_t launch_hexmv4(const HexArgs& a, hipStream_t stream);
@@ -525,8 +540,8 @@ int attention_static_error(int* was_set);
 // GSD_ATTN_SPIN_LIMIT -> spin_limit); both unset in use.
 void attention_test_knobs(AttnArgs& a);
 
-struct StepState {
-    int token;
+struct alignas(8) StepState {
+    int token;          // (token and pos are read as one word from host memory)
     int pos;
     int gen_count;
     int margin_bits;    // top1 - top2 of the last argmax (float bits)

@@ -1,24 +1,9 @@
 // gsd_kernels.hip -- gfx950 kernels of the GSD-LQ decode engine.
 //
-// Hot path: hexmv, the fused unpack + dequant matvec of GSD-LQ packed weights
-// (reference semantics: gsd_cpu_hex2d_matvec, gsd_lq_cpu_engine.c:129-183).
-// Design for CDNA4 (wave64, 160 KB LDS, HBM3E):
-//   * each thread owns fixed 32-column "slots" of the input vector and keeps
-//     that slice in VGPRs for the whole launch, so x is read once per block,
-//     not once per row;
-//   * for every row a slot is one 16-byte global load of codes (16 pairs),
-//     adjacent lanes read adjacent 16-byte pieces of the same row, so a wave
-//     reads 1 KB contiguous per row: 128-bit, fully coalesced;
-//   * codes are expanded through the codebook held in LDS (float2 per code),
-//     multiplied with the register-resident x slice in fp32, scaled once per
-//     16 pairs by the fp16 block scale;
-//   * RB rows are in flight per thread (RB independent 16-byte loads and FMA
-//     chains), reduced across the block with cross-lane shuffles + LDS;
-//   * prologue fusions: RMSNorm of the input (each block, from its register
-//     slice); the rank-k projection tmp_k = S * (Vt x) is computed once, by
-//     blocks 0..sum(k)-1, and published to the others through flags;
-//   * epilogue fusions: kinks and the U tmp_k term, then store / residual add /
-//     SwiGLU of paired gate-up rows.
+// The decode path's fused matvecs (hexmv4), attention, greedy step, the batched
+// projection on 16 x 16 tiles, and the operator twins (hexmv_file: the fused
+// unpack + dequant matvec over the file's own layout, reference semantics:
+// gsd_cpu_hex2d_matvec, gsd_lq_cpu_engine.c:129-183).
 #include <algorithm>
 #include <cstdlib>
 
@@ -29,486 +14,157 @@ namespace gsd {
 namespace {
 
 
-// 16 codes (one 16-byte load) against the 32 matching x values.
-__device__ __forceinline__ float dot16(const uint4 c, const float2* __restrict__ T, const float* xv) {
-    float p = 0.f;
-    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const float2 t = T[(w[d] >> (8 * b)) & 0xFFu];
-            p = fmaf(t.x, xv[8 * d + 2 * b], p);
-            p = fmaf(t.y, xv[8 * d + 2 * b + 1], p);
-        }
-    }
-    return p;
-}
-
-// Lattice form of dot16: with codeword (r0 + r1/2, r1*s), s = sqrt(3)/2, a pair
-// contributes xa*(r0 + r1/2) + xb*r1*s = u*r0 + v*r1 with u = xa and
-// v = xa/2 + s*xb precomputed per column pair (uv holds u, v interleaved).
-// The table entry is (r0, r1) as two fp16 (exact integers), so each pair is
-// one byte-select address (v_lshlrev_b32 SDWA), one 4-byte LDS read and two
-// mixed-precision FMAs (v_fma_mix_f32), all arithmetic in fp32.
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ float dot16_lat(const uint4 c, const half2v* __restrict__ T, const float* uv) {
-    float p0 = 0.f, p1 = 0.f;   // r0 and r1 terms: two independent FMA chains
-    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const half2v t = T[(w[d] >> (8 * b)) & 0xFFu];
-            p0 = fmaf((float)t.x, uv[8 * d + 2 * b], p0);
-            p1 = fmaf((float)t.y, uv[8 * d + 2 * b + 1], p1);
-        }
-    }
-    return p0 + p1;
-}
-
-// Cross-lane reduction of 8 per-lane partial sums (one per row of a batch)
-// with VALU permutes only: two swap-and-add rounds (v_permlane32_swap,
-// v_permlane16_swap) halve the values per lane while doubling their span,
-// then DPP adds finish each 16-lane row.  On return, lane 16q holds the
-// wave totals of rows 2q (u0) and 2q+1 (u1), q = 0..3.
-__device__ __forceinline__ void reduce8(const float (&acc)[8], float& u0, float& u1) {
-    const float t0 = swap_add32(acc[0], acc[4], false);   // rows 0 | 4
-    const float t1 = swap_add32(acc[1], acc[5], false);   // rows 1 | 5
-    const float t2 = swap_add32(acc[2], acc[6], false);   // rows 2 | 6
-    const float t3 = swap_add32(acc[3], acc[7], false);   // rows 3 | 7
-    u0 = row16_sum(swap_add16(t0, t2));                   // rows 0 | 2 | 4 | 6 per 16 lanes
-    u1 = row16_sum(swap_add16(t1, t3));                   // rows 1 | 3 | 5 | 7
-}
-
-// Rows of batch b.  Unpaired: RB consecutive rows of one segment.  Paired
-// (gate/up + SwiGLU): rows 0-3 of the batch are gate rows r0..r0+3, rows 4-7
-// the same rows of up.
-struct BatchRows {
-    int g0, r0;
-};
-
-// Rank-k value `lead` of a launch (segments in order, tmp_k == null ones only):
-// tmp_k[j] = S[j] * sum_c ((x[c] * inv) * w[c]) * Vt[j][c]
-// (gsd_lq_cpu_engine.c:66-82 then :110-127), published as one 64-bit word.
-// All loads of a thread (x, norm weights, Vt) are issued before any is used.
-template <int SPT>
-__device__ void lowrank_publish(const HexArgs& a, int lead, float* scratch) {
-    int g = 0, jj = lead;
-    for (; g < a.nseg; g++) {
-        const int k = a.seg[g].tmp_k ? 0 : a.seg[g].k;
-        if (jj < k) break;
-        jj -= k > 0 ? k : 0;
-    }
-    const HexSeg& sg = a.seg[g];
-    const int tid = threadIdx.x, NT = blockDim.x, S = a.cols >> 5;
-    float ss = 0.f, d = 0.f;
-    float4 xv[SPT][8], wv[SPT][8];
-    uint4 vv[SPT][4];
-#pragma unroll
-    for (int j = 0; j < SPT; j++) {
-        const int s = min(tid + j * NT, S - 1);
-        const float4* xp = reinterpret_cast<const float4*>(a.x + (size_t)s * 32);
-        const float4* wp = reinterpret_cast<const float4*>(a.norm_w ? a.norm_w + (size_t)s * 32 : a.x);
-        const uint4* vp = reinterpret_cast<const uint4*>(sg.Vt + (size_t)jj * a.cols + (size_t)s * 32);
-#pragma unroll
-        for (int q = 0; q < 8; q++) xv[j][q] = xp[q];
-        if (a.norm_w) {
-#pragma unroll
-            for (int q = 0; q < 8; q++) wv[j][q] = wp[q];
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) vv[j][q] = vp[q];
-    }
-#pragma unroll
-    for (int j = 0; j < SPT; j++) {
-        if (tid + j * NT >= S) continue;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            ss = fmaf(xv[j][q].x, xv[j][q].x, ss); ss = fmaf(xv[j][q].y, xv[j][q].y, ss);
-            ss = fmaf(xv[j][q].z, xv[j][q].z, ss); ss = fmaf(xv[j][q].w, xv[j][q].w, ss);
-        }
-    }
-    float inv = 1.f;
-    if (a.norm_w) {
-        ss = block_sum(ss, scratch);
-        inv = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
-    }
-#pragma unroll
-    for (int j = 0; j < SPT; j++) {
-        if (tid + j * NT >= S) continue;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            float xe[4] = {xv[j][q].x, xv[j][q].y, xv[j][q].z, xv[j][q].w};
-            if (a.norm_w) {
-                const float we[4] = {wv[j][q].x, wv[j][q].y, wv[j][q].z, wv[j][q].w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) xe[e] = (xe[e] * inv) * we[e];
-            }
-            const uint32_t h0 = (&vv[j][q >> 1].x)[2 * (q & 1)], h1 = (&vv[j][q >> 1].x)[2 * (q & 1) + 1];
-            d = fmaf(xe[0], h2f((uint16_t)(h0 & 0xFFFFu)), d);
-            d = fmaf(xe[1], h2f((uint16_t)(h0 >> 16)), d);
-            d = fmaf(xe[2], h2f((uint16_t)(h1 & 0xFFFFu)), d);
-            d = fmaf(xe[3], h2f((uint16_t)(h1 >> 16)), d);
-        }
-    }
-    d = block_sum(d, scratch);
-    if (tid == 0)
-        __hip_atomic_store(&a.pub[lead], (1ull << 32) | __float_as_uint(d * sg.S[jj]), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// TM: 0 = generic float2 codeword tables (one per segment), 1 = lattice
-// fields, one table shared by all segments, 2 = lattice fields per segment.
-template <int SPT, int NWM, bool ST, int TM>
-__global__ void __launch_bounds__(NWM * 64) hexmv_kernel(const HexArgs a) {
-    constexpr int RB = 8;
-    __shared__ float2 tbl[kMaxSeg][kTableSlots];   // TM > 0: half2 entries, 256 per segment
-    __shared__ float red[2][NWM][RB];
-    __shared__ float fin[RB];
-    __shared__ float tkl[kMaxSeg][kMaxRank];
-    __shared__ float scratch[16];
-    __shared__ float s_inv;
-
-    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wid = tid >> 6;
-    const int NW = NT >> 6;
-    const int S = a.cols >> 5;
-    const int nsb = a.cols >> 6;
+// ------------------------------------------------------------------------
+// Fused unpack + dequant matvec over the .gsd2 file layout, any codebook of
+// up to 256 float2 points (gsdh_hex2d_matvec).  A block owns 8 rows: 8 waves,
+// two sets of four rows, each row's columns over the four waves of its set; a
+// lane holds 16 columns of x in registers and loads 8 codes (8 bytes) of each
+// of its rows.  The wave's lanes also form one row's kink and U tmp_k terms,
+// whose three dependent loads then run beside the codebook's staging.
+// Bound: the launch's chain of round trips (codes, x and codebook together,
+// then the products, then the row sums), and the codebook lookups: 32 copies
+// of each point (64 KB), one per lane of a half wave, so that no two lanes of
+// a read share a bank; one shared copy cost 5-6 bank passes per read.
+// Measured (MI355X, 4096 x 4096, radius 6, a kink per row, rank 2): 9.1 us
+// with one copy, two waves per block over the row's full width and the kinks
+// after the row sums.
+// ------------------------------------------------------------------------
+__global__ void __launch_bounds__(512) hexmv_file_kernel(const FileMatvec a) {
+    __shared__ __attribute__((aligned(16))) float2 tab[kTableSlots * 32];   // entry e, copy c at 32 e + c
+    __shared__ float red[4][8], extra[8];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, rs = wid >> 2, cq = wid & 3;
+    const int slots = a.cols >> 4, nsb = a.cols >> 6;
     const size_t rowbytes = (size_t)(a.cols >> 1);
-    const bool paired = a.epilogue == kEpiSwiGLU;
-
-    auto rows_of = [&](int b) {
-        BatchRows br;
-        if (paired) {
-            br.g0 = 0;
-            br.r0 = b * (RB / 2);
-        } else {
-            int g = 0;
-            while (g + 1 < a.nseg && b >= a.seg[g + 1].batch0) g++;
-            br.g0 = g;
-            br.r0 = (b - a.seg[g].batch0) * RB;
+    const int row0 = (int)blockIdx.x * 8;
+    const uint8_t* cp[4];
+    const uint16_t* sp[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {   // (rows past the end: the last one's, not stored)
+        const size_t row = (size_t)min(row0 + rs * 4 + r, a.rows - 1);
+        cp[r] = a.codes + row * rowbytes;
+        sp[r] = a.scales + row * nsb;
+    }
+    uint2 cw[4];
+    uint16_t sv[4];
+    float4 xv[4];
+    auto load = [&](int s) {
+        s = min(s, slots - 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            cw[r] = *reinterpret_cast<const uint2*>(cp[r] + (size_t)s * 8);
+            sv[r] = sp[r][s >> 2];
         }
-        return br;
+        const float4* xp = reinterpret_cast<const float4*>(a.x) + (size_t)s * 4;
+#pragma unroll
+        for (int q = 0; q < 4; q++) xv[q] = xp[q];
     };
-
-    uint4 cw[SPT][RB];
-    uint32_t sv[SPT][RB];
-    uint4 uw[2];   // epilogue threads: U row (k <= 16 fp16) of their row, fetched with the batch
-    // Issue every load of batch b: RB x SPT 16-byte code loads and the
-    // matching scales, rows and slots clamped in range (results of padding
-    // rows/slots are discarded later), no branches between the loads.
-    auto issue = [&](int b) {
-        const BatchRows br = rows_of(b);
-#pragma unroll
-        for (int j = 0; j < SPT; j++) {
-            const int s = min(tid + j * NT, S - 1);
-#pragma unroll
-            for (int rr = 0; rr < RB; rr++) {
-                const int g = paired ? (rr >> 2) : br.g0;
-                const int row = min(br.r0 + (paired ? (rr & 3) : rr), a.seg[g].rows - 1);
-                cw[j][rr] = *reinterpret_cast<const uint4*>(a.seg[g].codes + (size_t)row * rowbytes + (size_t)s * 16);
-                if (!ST) sv[j][rr] = a.seg[g].scales[(size_t)row * nsb + (s >> 1)];
-            }
-            if (j == 0 && tid < RB) {
-                const int g = paired ? (tid >> 2) : br.g0;
-                const int kk = a.seg[g].k;
-                if (kk > 0) {
-                    const int row = min(br.r0 + (paired ? (tid & 3) : tid), a.seg[g].rows - 1);
-                    const uint16_t* up = a.seg[g].U + (size_t)row * kk;
-                    // U rows are 2*k bytes: fetch as 16-bit loads into the two vectors
-                    uint16_t tmp[16];
-#pragma unroll
-                    for (int q = 0; q < 16; q++) tmp[q] = q < kk ? up[q] : (uint16_t)0;
-                    uw[0] = make_uint4(tmp[0] | (uint32_t)tmp[1] << 16, tmp[2] | (uint32_t)tmp[3] << 16,
-                                       tmp[4] | (uint32_t)tmp[5] << 16, tmp[6] | (uint32_t)tmp[7] << 16);
-                    uw[1] = make_uint4(tmp[8] | (uint32_t)tmp[9] << 16, tmp[10] | (uint32_t)tmp[11] << 16,
-                                       tmp[12] | (uint32_t)tmp[13] << 16, tmp[14] | (uint32_t)tmp[15] << 16);
-                }
-            }
-            if (ST) {
-#pragma unroll
-                for (int grp = 0; grp < 2; grp++) {
-                    const int g = paired ? grp : br.g0;
-                    const int ngrp = (a.seg[g].rows + 3) >> 2;
-                    const int rg = min((br.r0 >> 2) + (paired ? 0 : grp), ngrp - 1);
-                    const uint2 w = *reinterpret_cast<const uint2*>(a.seg[g].scales + ((size_t)rg * nsb + (s >> 1)) * 4);
-                    sv[j][4 * grp + 0] = w.x & 0xFFFFu;
-                    sv[j][4 * grp + 1] = w.x >> 16;
-                    sv[j][4 * grp + 2] = w.y & 0xFFFFu;
-                    sv[j][4 * grp + 3] = w.y >> 16;
-                }
-            }
-        }
-    };
-
-    // blocks 0..nlead-1 compute the rank-k projections and exit; the matvec
-    // blocks follow them
-    int nlead = 0;
-    for (int g = 0; g < a.nseg; g++)
-        if (!a.seg[g].tmp_k) nlead += a.seg[g].k > 0 ? a.seg[g].k : 0;
-    if ((int)blockIdx.x < nlead) {
-        lowrank_publish<SPT>(a, (int)blockIdx.x, scratch);
-        return;
+    const int s0 = cq * 64 + lane;
+    load(s0);
+    // the wave's own row (8 waves, 8 rows): CSR range and rank-k factors
+    const int krow = min(row0 + wid, a.rows - 1);
+    uint32_t e0 = 0, e1 = 0;
+    if (a.row_ptr) {
+        e0 = a.row_ptr[krow];
+        e1 = a.row_ptr[krow + 1];
     }
-    const int nblk = (int)gridDim.x - nlead;
-    int b = (int)blockIdx.x - nlead;
-    if (b < a.nbatch) issue(b);   // in flight while the prologue runs
-
-    half2v* ltab = reinterpret_cast<half2v*>(&tbl[0][0]);
-    if (TM == 0) {
-        for (int g = 0; g < a.nseg; g++) {
-            const float2* tg = reinterpret_cast<const float2*>(a.seg[g].table);
-            for (int i = tid; i < kTableSlots; i += NT) tbl[g][i] = i < a.seg[g].n_pts ? tg[i] : make_float2(0.f, 0.f);
+    float ex = lane < a.k ? h2f(a.U[(size_t)krow * a.k + lane]) * a.tmp_k[lane] : 0.f;
+    // the codebook: thread (e, c) of each pass writes copy c of entry e
+    {
+        const int c = tid & 31;
+        float2 t[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int e = (tid >> 5) + 16 * i;
+            t[i] = e < a.n_pts ? a.table[e] : make_float2(0.f, 0.f);
         }
-    } else {
-        for (int g = 0; g < (TM == 1 ? 1 : a.nseg); g++) {
-            const half2v* fg = reinterpret_cast<const half2v*>(a.seg[g].fields);
-            for (int i = tid; i < kTableSlots; i += NT) {
-                half2v z; z.x = (_Float16)0.f; z.y = (_Float16)0.f;
-                ltab[g * kTableSlots + i] = i < a.seg[g].n_pts ? fg[i] : z;
-            }
-        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) tab[((tid >> 5) + 16 * i) * 32 + c] = t[i];
     }
-
-    // input slice: slot s = tid + j*NT covers columns [32s, 32s+32)
-    float xr[SPT][32];
-#pragma unroll
-    for (int j = 0; j < SPT; j++) {
-        const int s = tid + j * NT;
-        if (s < S) {
-            const float4* xp = reinterpret_cast<const float4*>(a.x + (size_t)s * 32);
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const float4 v = xp[q];
-                xr[j][4 * q] = v.x; xr[j][4 * q + 1] = v.y; xr[j][4 * q + 2] = v.z; xr[j][4 * q + 3] = v.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 32; q++) xr[j][q] = 0.f;
-        }
-    }
-
-    // fused RMSNorm (gsd_lq_cpu_engine.c:66-82): x' = (x * inv) * w
-    float inv = 1.f;
-    if (a.norm_w) {
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < SPT; j++)
-#pragma unroll
-            for (int q = 0; q < 32; q++) ss = fmaf(xr[j][q], xr[j][q], ss);
-        ss = block_sum(ss, scratch);
-        inv = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
-#pragma unroll
-        for (int j = 0; j < SPT; j++) {
-            const int s = tid + j * NT;
-            if (s < S) {
-                const float4* wp = reinterpret_cast<const float4*>(a.norm_w + (size_t)s * 32);
-#pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    const float4 w = wp[q];
-                    xr[j][4 * q] = (xr[j][4 * q] * inv) * w.x;
-                    xr[j][4 * q + 1] = (xr[j][4 * q + 1] * inv) * w.y;
-                    xr[j][4 * q + 2] = (xr[j][4 * q + 2] * inv) * w.z;
-                    xr[j][4 * q + 3] = (xr[j][4 * q + 3] * inv) * w.w;
-                }
-            }
-        }
-    }
-    if (tid == 0) s_inv = inv;
-    if (TM != 0) {
-        // lattice path: (xa, xb) -> (u, v) = (xa, xa/2 + xb*sqrt(3)/2)
-        constexpr float kS32 = 0.866025403784438646763723170752936183f;
-#pragma unroll
-        for (int j = 0; j < SPT; j++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) xr[j][2 * q + 1] = fmaf(kS32, xr[j][2 * q + 1], 0.5f * xr[j][2 * q]);
-    }
-
-    // rank-k values: given (tmp_k, copied here) or published by the
-    // projection blocks (fetched by each epilogue lane when it first needs a
-    // segment's values; bit g of `have` marks segment g as fetched)
-    unsigned have = 0;
-    for (int g = 0; g < a.nseg; g++) {
-        if (a.seg[g].k > 0 && a.seg[g].tmp_k) {
-            if (tid < a.seg[g].k) tkl[g][tid] = a.seg[g].tmp_k[tid];
-            have |= 1u << g;
-        }
-    }
+    for (uint32_t i = e0 + lane; i < e1; i += 64) ex += a.kdel[i] * a.x[a.kcols[i]];
+    ex = wave_sum_valu(ex);
+    if (lane == 0) extra[wid] = ex;
     __syncthreads();
 
-    int buf = 0;
-    for (; b < a.nbatch; b += nblk) {
-        const BatchRows br = rows_of(b);
-        float acc[RB];
+    const unsigned char* tb = reinterpret_cast<const unsigned char*>(tab);
+    const uint32_t off = (uint32_t)(lane & 31) * 8u;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < slots; s += 256) {
+        uint32_t w[4][2];
+        float x[16], sc[4];
 #pragma unroll
-        for (int rr = 0; rr < RB; rr++) acc[rr] = 0.f;
+        for (int r = 0; r < 4; r++) {
+            w[r][0] = cw[r].x;
+            w[r][1] = cw[r].y;
+            sc[r] = h2f(sv[r]);
+        }
 #pragma unroll
-        for (int j = 0; j < SPT; j++) {
-            if (tid + j * NT < S) {
+        for (int q = 0; q < 4; q++) {
+            x[4 * q] = xv[q].x;
+            x[4 * q + 1] = xv[q].y;
+            x[4 * q + 2] = xv[q].z;
+            x[4 * q + 3] = xv[q].w;
+        }
+        if (s + 256 < slots) load(s + 256);
 #pragma unroll
-                for (int rr = 0; rr < RB; rr++) {
-                    const int g = paired ? (rr >> 2) : br.g0;
-                    float d;
-                    if (TM == 0) d = dot16(cw[j][rr], tbl[g], xr[j]);
-                    else d = dot16_lat(cw[j][rr], ltab + (TM == 1 ? 0 : g * kTableSlots), xr[j]);
-                    acc[rr] = fmaf(d, h2f((uint16_t)sv[j][rr]), acc[rr]);
-                }
+        for (int r = 0; r < 4; r++) {
+            float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {   // byte code << 8 | copy offset
+                const uint32_t ad = __builtin_amdgcn_perm(w[r][j >> 2], off, 0x0C0C0400u + ((uint32_t)(j & 3) << 8));
+                const float2 t = *reinterpret_cast<const float2*>(tb + ad);
+                p0 = fmaf(t.x, x[2 * j], p0);
+                p1 = fmaf(t.y, x[2 * j + 1], p1);
             }
+            acc[r] = fmaf(p0 + p1, sc[r], acc[r]);
         }
-        const uint4 uw_cur[2] = {uw[0], uw[1]};
-        // next batch's loads fly during the reduction and the epilogue
-        if (b + nblk < a.nbatch) issue(b + nblk);
-
-        float u0, u1;
-        reduce8(acc, u0, u1);
-        if ((lane & 15) == 0) {
-            red[buf][wid][2 * (lane >> 4)] = u0;
-            red[buf][wid][2 * (lane >> 4) + 1] = u1;
-        }
-        __syncthreads();
-        if (tid < RB) {
-            const int rr = tid;
-            const int g = paired ? (rr >> 2) : br.g0;
-            const int row = br.r0 + (paired ? (rr & 3) : rr);
-            const HexSeg& sg = a.seg[g];
-            float t = 0.f;
-            for (int w = 0; w < NW; w++) t += red[buf][w][rr];
-            if (row < sg.rows) {
-                if (sg.row_ptr) {
-                    const uint32_t e = sg.row_ptr[row + 1];
-                    for (uint32_t i = sg.row_ptr[row]; i < e; i++) {
-                        const int c = sg.kcols[i];
-                        const float xc = a.norm_w ? (a.x[c] * s_inv) * a.norm_w[c] : a.x[c];
-                        t += sg.kdel[i] * xc;
-                    }
-                }
-                if (sg.k > 0 && !((have >> g) & 1u)) {
-                    // this segment's published words (segments without tmp_k
-                    // in order); a bounded wait, normally already satisfied:
-                    // after 2^20 polls the error word is set
-                    int off = 0;
-                    for (int g2 = 0; g2 < g; g2++)
-                        if (!a.seg[g2].tmp_k && a.seg[g2].k > 0) off += a.seg[g2].k;
-                    int spins = 0;
-                    for (int jj = 0; jj < sg.k; jj++) {
-                        unsigned long long w;
-                        while (((w = __hip_atomic_load(&a.pub[off + jj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) == 0 &&
-                               spins < (1 << 20)) {
-                            if (++spins == (1 << 20)) *a.err = 1u;
-                            __builtin_amdgcn_s_sleep(1);
-                        }
-                        tkl[g][jj] = __uint_as_float((unsigned)w);
-                    }
-                    have |= 1u << g;
-                }
-                const uint32_t uu[8] = {uw_cur[0].x, uw_cur[0].y, uw_cur[0].z, uw_cur[0].w,
-                                        uw_cur[1].x, uw_cur[1].y, uw_cur[1].z, uw_cur[1].w};
-                for (int jj = 0; jj < sg.k; jj++) t += h2f((uint16_t)(uu[jj >> 1] >> (16 * (jj & 1)))) * tkl[g][jj];
-                if (a.epilogue == kEpiStore) sg.out[row] = t;
-                else if (a.epilogue == kEpiResidual) a.resid[row] = a.resid[row] + t;
-            }
-            fin[rr] = t;
-        }
-        if (a.epilogue == kEpiRopeKV) {
-            // segments q, k, v; rows 2i, 2i+1 of a head are one rotation pair
-            // (interleaved RoPE, gsd_lq_cpu_engine.c:213-256), evaluated without
-            // contraction like the reference; k', v stored as fp16 at pos
-            __syncthreads();
-            if (tid < RB / 2) {
-#pragma clang fp contract(off)
-                const RopeKV& r = a.rope;
-                const int row = br.r0 + 2 * tid;
-                const HexSeg& sg = a.seg[br.g0];
-                if (row + 1 < sg.rows) {
-                    const int pos = r.pos_dev ? *r.pos_dev : r.pos;
-                    const float x0 = fin[2 * tid], x1 = fin[2 * tid + 1];
-                    const size_t base = ((size_t)r.layer * r.max_seq + (size_t)pos) * (size_t)r.n_kv * r.hd;
-                    if (br.g0 == 2) {
-                        r.v_cache[base + row] = f2h(x0);
-                        r.v_cache[base + row + 1] = f2h(x1);
-                    } else {
-                        const float2 cs = r.cs[(size_t)pos * (r.hd >> 1) + ((row % r.hd) >> 1)];
-                        const float y0 = x0 * cs.x - x1 * cs.y;
-                        const float y1 = x0 * cs.y + x1 * cs.x;
-                        if (br.g0 == 0) {
-                            sg.out[row] = y0;
-                            sg.out[row + 1] = y1;
-                        } else {
-                            r.k_cache[base + row] = f2h(y0);
-                            r.k_cache[base + row + 1] = f2h(y1);
-                        }
-                    }
-                }
-            }
-        }
-        if (paired) {
-            __syncthreads();
-            if (tid < RB / 2) {
-                const int row = br.r0 + tid;
-                if (row < a.seg[0].rows) {
-                    const float gt = fin[tid], up = fin[tid + RB / 2];
-                    a.seg[0].out[row] = (gt / (1.0f + expf(-gt))) * up;
-                }
-            }
-        }
-        buf ^= 1;
     }
-}
-
-template <int SPT, int NWM, bool ST, int TM>
-hipError_t launch_hexmv_t(const HexArgs& a, hipStream_t st, int nt) {
-    constexpr int RB = 8;
-    HexArgs b = a;
-    if (b.epilogue == kEpiSwiGLU) {
-        b.nbatch = (b.seg[0].rows + RB / 2 - 1) / (RB / 2);
-    } else {
-        int nb = 0;
-        for (int g = 0; g < b.nseg; g++) {
-            b.seg[g].batch0 = nb;
-            nb += (b.seg[g].rows + RB - 1) / RB;
-        }
-        b.nbatch = nb;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float t = wave_sum_valu(acc[r]);
+        if (lane == 0) red[cq][rs * 4 + r] = t;
     }
-    if (b.nbatch == 0) return hipSuccess;
-    // persistent grid: as many blocks as are resident on the chip at once
-    static int per_cu = 0;
-    if (per_cu == 0) {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, hexmv_kernel<SPT, NWM, ST, TM>, nt, 0) != hipSuccess || n < 1)
-            n = 1;
-        per_cu = n;
-    }
-    // persistent grid (as many blocks as are resident, each looping over
-    // batches with the next batch's loads in flight); GSD_HEXMV_PERSIST=0
-    // launches one block per batch instead
-    static const int persist = getenv("GSD_HEXMV_PERSIST") ? atoi(getenv("GSD_HEXMV_PERSIST")) : 1;
-    const int ncu = device_cu_count() > 0 ? device_cu_count() : 256;
-    // blocks 0..nlead-1 publish the rank-k values and exit after one short
-    // pass; the matvec blocks follow them (dispatched in order, so a matvec
-    // block never waits on a publishing block that is not yet resident)
-    int nlead = 0;
-    for (int g = 0; g < b.nseg; g++)
-        if (!b.seg[g].tmp_k && b.seg[g].k > 0) nlead += b.seg[g].k;
-    if (nlead > 0 && (!b.pub || !b.err)) return hipErrorInvalidValue;
-    int grid = persist ? ncu * per_cu : b.nbatch;
-    if (grid > b.nbatch) grid = b.nbatch;
-    grid += nlead;
-    hipLaunchKernelGGL((hexmv_kernel<SPT, NWM, ST, TM>), dim3(grid), dim3(nt), 0, st, b);
-    return hipGetLastError();
+    __syncthreads();
+    if (tid < 8 && row0 + tid < a.rows) a.y[row0 + tid] = ((red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid])) + extra[tid];
 }
 
 // ------------------------------------------------------------------------
 // rank-k projection twin: one block per j
 // ------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) lowrank_kernel(const float* x, const uint16_t* Vt, const float* S,
-                                                      float* tmp_k, int cols) {
+// VEC: rows of x and Vt in 16- and 8-byte loads, four in flight per thread
+// (4096 columns: one round; 3.8 us with 256 threads of scalar loads)
+template <bool VEC>
+__global__ void __launch_bounds__(1024) lowrank_kernel(const float* x, const uint16_t* Vt, const float* S,
+                                                       float* tmp_k, int cols) {
     __shared__ float scratch[16];
-    const int j = blockIdx.x;
+    const int j = blockIdx.x, tid = threadIdx.x;
+    const uint16_t* vt = Vt + (size_t)j * cols;
     float p = 0.f;
-    for (int c = threadIdx.x; c < cols; c += blockDim.x) p = fmaf(x[c], h2f(Vt[(size_t)j * cols + c]), p);
+    if (VEC) {
+        const float4* x4 = reinterpret_cast<const float4*>(x);
+        const uint2* v4 = reinterpret_cast<const uint2*>(vt);
+        const int n = cols >> 2;
+        for (int c = tid; c < n; c += 4096) {
+            float4 xv[4];
+            uint2 vv[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const bool ok = c + 1024 * q < n;
+                xv[q] = ok ? x4[c + 1024 * q] : make_float4(0.f, 0.f, 0.f, 0.f);
+                vv[q] = ok ? v4[c + 1024 * q] : make_uint2(0u, 0u);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                p = fmaf(xv[q].x, h2f((uint16_t)(vv[q].x & 0xFFFFu)), p);
+                p = fmaf(xv[q].y, h2f((uint16_t)(vv[q].x >> 16)), p);
+                p = fmaf(xv[q].z, h2f((uint16_t)(vv[q].y & 0xFFFFu)), p);
+                p = fmaf(xv[q].w, h2f((uint16_t)(vv[q].y >> 16)), p);
+            }
+        }
+    } else {
+        for (int c = tid; c < cols; c += 1024) p = fmaf(x[c], h2f(vt[c]), p);
+    }
     p = block_sum(p, scratch);
-    if (threadIdx.x == 0) tmp_k[j] = p * S[j];
+    if (tid == 0) tmp_k[j] = p * S[j];
 }
 
 __global__ void __launch_bounds__(1024) rmsnorm_kernel(const float* x, const float* w, float* out, int dim, float eps) {
@@ -1471,17 +1127,24 @@ __global__ void set_step_kernel(StepState* st, int token, int pos, int reset_err
 
 // host_in (pinned host memory, or null): the step's token and position, which
 // the launch also puts into the step state; else the state's own token
-__global__ void embed_kernel(const uint16_t* embed, StepState* st, const StepState* host_in, float* x, int hidden,
+__global__ void __launch_bounds__(1024) embed_kernel(const uint16_t* embed, StepState* st, const StepState* host_in, float* x, int hidden,
                              unsigned long long* clear, int nclear, unsigned* epoch) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int token;
-    if (host_in) {
-        token = __hip_atomic_load(&host_in->token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (i == 0) {
-            *st = StepState{};
-            st->token = token;
-            st->pos = __hip_atomic_load(&host_in->pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (host_in) {   // one lane per block reads over PCIe (every wave doing so: 10.4 us for the launch, so 5.2)
+        __shared__ int tk;
+        if (threadIdx.x == 0) {
+            const unsigned long long w = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(host_in),
+                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // token | pos << 32
+            tk = (int)(unsigned)w;
+            if (blockIdx.x == 0) {
+                *st = StepState{};
+                st->token = (int)(unsigned)w;
+                st->pos = (int)(unsigned)(w >> 32);
+            }
         }
+        __syncthreads();
+        token = tk;
     } else {
         token = st->token;
     }
@@ -3571,40 +3234,10 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const PrefillAttn a) 
 // ------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------
-hipError_t launch_hexmv(const HexArgs& a, hipStream_t st) {
-    const int S = a.cols >> 5;
-    // one 32-column slot per thread (fewest VGPRs, most waves per CU); two
-    // when the row has more than 1024 slots
-    const int spt = S <= 1024 ? 1 : 2;
-    const int nt = ((S + spt - 1) / spt + 63) / 64 * 64;
-    if (nt > 1024) return hipErrorInvalidValue;
-    bool lattice = a.nseg > 0, shared = true;
-    for (int g = 0; g < a.nseg; g++) {
-        lattice = lattice && a.seg[g].fields != nullptr;
-        shared = shared && a.seg[g].fields == a.seg[0].fields && a.seg[g].n_pts == a.seg[0].n_pts;
-    }
-    // lattice fields come with the 4-row scale groups; the generic path
-    // reads the file's row-major scales
-    if (lattice != (a.scale_t != 0)) return hipErrorInvalidValue;
-#define GSD_HEXMV_DISPATCH(ST, TM)                                                  \
-    if (spt == 2) {                                                                 \
-        if (nt <= 64) return launch_hexmv_t<2, 1, ST, TM>(a, st, nt);                \
-        if (nt <= 256) return launch_hexmv_t<2, 4, ST, TM>(a, st, nt);               \
-        if (nt <= 512) return launch_hexmv_t<2, 8, ST, TM>(a, st, nt);               \
-        return launch_hexmv_t<2, 16, ST, TM>(a, st, nt);                             \
-    }                                                                               \
-    if (nt <= 64) return launch_hexmv_t<1, 1, ST, TM>(a, st, nt);                    \
-    if (nt <= 256) return launch_hexmv_t<1, 4, ST, TM>(a, st, nt);                   \
-    if (nt <= 512) return launch_hexmv_t<1, 8, ST, TM>(a, st, nt);                   \
-    return launch_hexmv_t<1, 16, ST, TM>(a, st, nt);
-    if (!lattice) {
-        GSD_HEXMV_DISPATCH(false, 0)
-    } else if (shared) {
-        GSD_HEXMV_DISPATCH(true, 1)
-    } else {
-        GSD_HEXMV_DISPATCH(true, 2)
-    }
-#undef GSD_HEXMV_DISPATCH
+hipError_t launch_hexmv_file(const FileMatvec& a, hipStream_t st) {
+    if (a.rows <= 0) return hipSuccess;
+    hipLaunchKernelGGL(hexmv_file_kernel, dim3((a.rows + 7) / 8), dim3(512), 0, st, a);
+    return hipGetLastError();
 }
 
 // Half units of a paired launch (GSD_GATEUP_HALVES=0 turns them off, to
@@ -3974,7 +3607,9 @@ hipError_t launch_lowrank_batched(const uint16_t* X, const uint16_t* Vt, const f
 hipError_t launch_lowrank(const float* x, const uint16_t* Vt, const float* S, float* tmp_k, int k, int cols,
                           hipStream_t st) {
     if (k <= 0) return hipSuccess;
-    hipLaunchKernelGGL(lowrank_kernel, dim3(k), dim3(256), 0, st, x, Vt, S, tmp_k, cols);
+    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(Vt) & 7) == 0;
+    if (vec) hipLaunchKernelGGL(lowrank_kernel<true>, dim3(k), dim3(1024), 0, st, x, Vt, S, tmp_k, cols);
+    else hipLaunchKernelGGL(lowrank_kernel<false>, dim3(k), dim3(1024), 0, st, x, Vt, S, tmp_k, cols);
     return hipGetLastError();
 }
 
@@ -4152,8 +3787,8 @@ hipError_t launch_prefill_attention(const PrefillAttn& a, hipStream_t st) {
 
 hipError_t launch_embed(const uint16_t* embed, StepState* stt, const StepState* host_in, float* x, int hidden,
                         unsigned long long* clear, int nclear, unsigned* epoch, hipStream_t st) {
-    const int n = hidden > nclear ? hidden : nclear;
-    hipLaunchKernelGGL(embed_kernel, dim3((n + 255) / 256), dim3(256), 0, st, embed, stt, host_in, x, hidden, clear,
+    const int n = hidden > nclear ? hidden : nclear, nt = host_in ? 1024 : 256;
+    hipLaunchKernelGGL(embed_kernel, dim3((n + nt - 1) / nt), dim3(nt), 0, st, embed, stt, host_in, x, hidden, clear,
                        nclear, epoch);
     return hipGetLastError();
 }

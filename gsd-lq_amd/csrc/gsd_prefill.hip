@@ -219,10 +219,11 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
             for (int g = 0; g < T2; g++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) d[r & 1][g][i] = 0.f;
+            // (low parts first: the block's sum is rounded while it is small)
 #pragma unroll
-            for (int s = 0; s < 4; s++)
+            for (int hl = NH - 1; hl >= 0; hl--)
 #pragma unroll
-                for (int hl = 0; hl < NH; hl++)
+                for (int s = 0; s < 4; s++)
 #pragma unroll
                     for (int g = 0; g < T2; g++)
                         d[r & 1][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[g][s][hl], bw[r & 1][s], d[r & 1][g], 0, 0, 0);
@@ -824,8 +825,8 @@ __global__ void __launch_bounds__(512, 2) attn_prompt_kernel(const PrefillAttn a
                     const uint2 lo4 = *reinterpret_cast<const uint2*>(vrow), hi4 = *reinterpret_cast<const uint2*>(vrow + 8);
                     const u32x4v vw = {lo4.x, lo4.y, hi4.x, hi4.y};
                     const half8v va = __builtin_bit_cast(half8v, vw);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph[st], o[d], 0, 0, 0);
                     o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl[st], o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph[st], o[d], 0, 0, 0);
                 }
             }
         }
