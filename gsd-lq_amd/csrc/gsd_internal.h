@@ -305,6 +305,7 @@ struct MmSeg {
     size_t p0;
     int rows, k, nsplit;
     int b0;                    // the tensor's first block (a multiple of 8)
+    int x0;                    // the XCD of its first row tile
 };
 // What a projection's result still needs of its input: the per-token descale
 // and, for the kink terms, the input itself (fp32, or bf16)

@@ -110,9 +110,10 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
     const MmSeg& w = a.seg[sg];
     const int rows = w.rows, nrb = (rows + 15) >> 4, n_rt = (nrb + RB - 1) / RB;
     // the token tiles and column splits of one row tile on one XCD (blocks
-    // go to the 8 XCDs in turn; b0 is a multiple of 8)
+    // go to the 8 XCDs in turn; b0 is a multiple of 8), the tensors' row tiles
+    // dealt on from XCD to XCD
     const int S = w.nsplit, cps = (nc + S - 1) / S, bl = (int)blockIdx.x - w.b0;
-    const int xcd = bl & 7, bq = bl >> 3;
+    const int xcd = (bl + 8 - w.x0) & 7, bq = bl >> 3;
     const int rt = (bq / (n_tt * S)) * 8 + xcd, tt = (bq % (n_tt * S)) / S, ks = bq % S;
     if (rt >= n_rt) return;
     const int rb0 = rt * RB + wid * R2 * 2, g0 = tt * TG;
@@ -316,6 +317,23 @@ __global__ void __launch_bounds__(256) mm_reduce_kernel(const MmArgs a) {
     }
 }
 
+// The token of a block of the two operand kernels, one block per token of ng
+// groups of 16, or -1 (a block of the last round's groups past the end).  The
+// 16 tokens of a group fill their lines of fragments 16 bytes each, so from 8
+// groups on a group's blocks are on one XCD, whose L2 joins them (a 411-token
+// chunk in block order wrote them from all 8: SwiGLU row of 14336 31 us
+// against 26 for 512 tokens); fewer groups spread over the XCDs instead.
+__device__ __forceinline__ int token_of_block(int ng) {
+    const int b = (int)blockIdx.x;
+    if (ng < 8) return b;
+    const int j = b >> 3, g = (j >> 4) * 8 + (b & 7);
+    return g < ng ? g * 16 + (j & 15) : -1;
+}
+dim3 token_grid(int M) {
+    const int ng = (M + 15) / 16;
+    return dim3(ng < 8 ? ng * 16 : (ng + 7) / 8 * 128);
+}
+
 // ------------------------------------------------------------------------
 // Operands of the next projections from what the last launch left: the
 // token's row (IN 0: X; 1: X plus the last projection, written back; 2:
@@ -331,19 +349,14 @@ __global__ void __launch_bounds__(256) mm_reduce_kernel(const MmArgs a) {
 // (13.5 us), a SwiGLU launch (15.8 us) and this pass reading their results
 // (11-24 us).
 // ------------------------------------------------------------------------
-template <int IN>
-__global__ void __launch_bounds__(512) layer_prep_kernel(const LayerPrep p) {
+template <int IN, int NT>
+__global__ void __launch_bounds__(NT) layer_prep_kernel(const LayerPrep p) {
     extern __shared__ __attribute__((aligned(16))) float xl[];   // the token's row
-    __shared__ float red[8][2 * kMaxSeg + 2];
+    __shared__ float red[NT / 64][2 * kMaxSeg + 2];
     constexpr float kS32 = 0.866025403784438646763723170752936183f;
-    constexpr int NT = 512, NS = 2 * kMaxSeg;
-    // the 16 rows of a token group, whose fragments share lines, on one XCD
-    // (the identity unless the groups divide evenly)
-    int m = (int)blockIdx.x;
-    if (!(gridDim.x & 127)) {
-        const int x = m & 7, j = m >> 3;
-        m = ((j >> 4) * 8 + x) * 16 + (j & 15);
-    }
+    constexpr int NS = 2 * kMaxSeg;
+    const int m = token_of_block((p.M + 15) >> 4);
+    if (m < 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int cols = p.cols, nc = (cols + 127) >> 7, np = cols >> 1, nv4 = cols >> 2;
     const bool valid = m < p.M;
@@ -548,11 +561,8 @@ __global__ void __launch_bounds__(512) mm_xprep_kernel(const MmXprep p) {
     constexpr int NS = 2 * kMaxSeg;
     __shared__ float red[8][NS + 1];
     constexpr float kS32 = 0.866025403784438646763723170752936183f;
-    int m = (int)blockIdx.x;
-    if (!(gridDim.x & 127)) {   // a token group's rows on one XCD
-        const int x = m & 7, j = m >> 3;
-        m = ((j >> 4) * 8 + x) * 16 + (j & 15);
-    }
+    const int m = token_of_block((p.M + 15) >> 4);
+    if (m < 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int nc = (p.cols + 127) >> 7, ng8 = p.cols >> 3;
     const bool valid = m < p.M;
@@ -960,12 +970,15 @@ MmTile hexmm32_tile(int M, int rows, int cols) {
     return t;
 }
 
-// Fills seg[].b0, .nsplit and .p0 for the tile; returns the floats of partial
+// Fills seg[].b0, .x0, .nsplit and .p0 for the tile; returns the floats of partial
 // sums (seg[].rows set).  Tensors of one launch that are split differently
-// keep their own split (nsplit 0: the tile's).
+// keep their own split (nsplit 0: the tile's).  A tensor's row tiles begin on
+// the XCD after the last tensor's end: with every tensor's from XCD 0 on, the
+// four row tiles each of k and v (7B shape, 512 tokens) kept four XCDs busy
+// while the others waited (q, k, v: 70 us against 49; k and v alone 50, 29).
 size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid) {
     const int ng = (a.M + 15) / 16, n_tt = (ng + 2 * t.t2 - 1) / (2 * t.t2);
-    int b = 0;
+    int b = 0, x = 0;
     size_t p = 0;
     a.r2 = t.r2;
     a.t2 = t.t2;
@@ -974,8 +987,10 @@ size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid) {
         if (w.nsplit <= 0) w.nsplit = t.nsplit;
         const int n_rt = ((w.rows + 15) / 16 + 8 * t.r2 - 1) / (8 * t.r2);
         w.b0 = b;
+        w.x0 = x;
         w.p0 = p;
         b += 8 * n_tt * w.nsplit * ((n_rt + 7) / 8);
+        x = (x + n_rt) & 7;
         if (w.nsplit > 1) p += (size_t)w.nsplit * ng * 16 * w.rows;
     }
     *grid = b;
@@ -1017,26 +1032,30 @@ bool mm_xprep_covers(const MmXprep& p) {
 
 hipError_t launch_mm_xprep(const MmXprep& p, hipStream_t st) {
     if (p.M <= 0 || p.cols <= 0 || p.cols % 64 || !p.X || !p.xa || !p.xs || !mm_xprep_covers(p)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(mm_xprep_kernel, dim3(((p.M + 15) / 16) * 16), dim3(512), 0, st, p);
+    hipLaunchKernelGGL(mm_xprep_kernel, token_grid(p.M), dim3(512), 0, st, p);
     return hipGetLastError();
 }
 
 hipError_t launch_layer_prep(const LayerPrep& p, LayerPrepIn in, hipStream_t st) {
     if (p.M <= 0 || p.cols <= 0 || p.cols % 64 || p.cols > kLayerPrepMaxCols || !p.xa || !p.xs) return hipErrorInvalidValue;
     const size_t lds = (size_t)p.cols * 4;
-    const dim3 grid(((p.M + 15) / 16) * 16);
-#define GSD_PREP(IN)                                                                                                     \
+    const dim3 grid = token_grid(p.M);
+    // up to a block per CU: 16 waves each, for the loads in flight (37 tokens,
+    // SwiGLU row of 14336: 20.4 -> 15.0 us); more blocks share the CUs and
+    // are faster with 8 (512 tokens: 26.8 against 30.6, 304: 24.1 both)
+    const bool wide = (int)grid.x <= (device_cu_count() > 0 ? device_cu_count() : 256);
+#define GSD_PREP_N(IN, NT)                                                                                               \
     {                                                                                                                    \
         static size_t attr = 0;                                                                                          \
         if (lds > attr) {                                                                                                \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&layer_prep_kernel<IN>),              \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&layer_prep_kernel<IN, NT>),          \
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);              \
             if (e != hipSuccess) return e;                                                                               \
             attr = lds;                                                                                                  \
         }                                                                                                                \
-        hipLaunchKernelGGL((layer_prep_kernel<IN>), grid, dim3(512), lds, st, p);                                        \
-        break;                                                                                                           \
+        hipLaunchKernelGGL((layer_prep_kernel<IN, NT>), grid, dim3(NT), lds, st, p);                                     \
     }
+#define GSD_PREP(IN) if (wide) GSD_PREP_N(IN, 1024) else GSD_PREP_N(IN, 512) break;
     switch (in) {
         case kPrepRow: GSD_PREP(0)
         case kPrepResidual: GSD_PREP(1)
@@ -1044,6 +1063,7 @@ hipError_t launch_layer_prep(const LayerPrep& p, LayerPrepIn in, hipStream_t st)
         case kPrepEmbed: GSD_PREP(3)
     }
 #undef GSD_PREP
+#undef GSD_PREP_N
     return hipGetLastError();
 }
 
