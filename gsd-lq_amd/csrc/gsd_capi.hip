@@ -1646,7 +1646,7 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
     auto flush = [&]() -> int {
         if (!a.nseg) return 0;
         int grid = 0;
-        (void)hexmm32_layout(a, MmTile{a.r2, a.t2, 1}, &grid);
+        (void)hexmm32_layout(a, MmTile{a.nw, a.t2, 1}, &grid);
         HIPCHK(launch_hexmm32(a, grid, m->stream));
         HIPCHK(launch_mm_reduce(a, m->stream));
         a.nseg = 0;
@@ -1660,7 +1660,7 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
                                                                                                     : MmTile{};
         if (tile.nsplit > 0) {
             if (a.nseg && a.n_pts != n_pts && (rc = flush())) return rc;
-            a.n_pts = n_pts; a.fields = m->fields[t.radius]; a.r2 = tile.r2; a.t2 = tile.t2;
+            a.n_pts = n_pts; a.fields = m->fields[t.radius]; a.nw = tile.nw; a.t2 = tile.t2;
             MmSeg& sg = a.seg[a.nseg++];
             sg = mm_seg(t, Y[i]);
             sg.nsplit = tile.nsplit;
@@ -1686,7 +1686,7 @@ int gsdh_matmul_plan(int M, int rows, int cols, int* tg, int* rbw, int* nsplit) 
     const MmTile t = hexmm32_tile(M, rows, cols);
     if (t.nsplit > 0) {   // 16-token groups per block, 16-row blocks per wave
         *tg = 2 * t.t2;
-        *rbw = 2 * t.r2;
+        *rbw = 2;
         *nsplit = t.nsplit;
         return 0;
     }

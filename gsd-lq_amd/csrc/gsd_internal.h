@@ -220,7 +220,7 @@ struct FileMatvec {
 };
 hipError_t launch_hexmv_file(const FileMatvec& a, hipStream_t stream);
 // MFMA matvec over the tiled layout (codes_t / scales_t / fields of every
-// segment); same epilogues, norm and rank-k handling as launch_hexmv.
+// segment), epilogues, norm and rank-k terms as HexArgs says.
 hipError_t launch_hexmv4(const HexArgs& a, hipStream_t stream);
 
 // Batched projection (prefill) on the matrix cores: Y[m][r] = W x_m for M
@@ -318,14 +318,14 @@ struct MmIn {
 struct MmArgs {
     MmSeg seg[kMaxSeg];
     int nseg, n_pts, M, hl, accumulate;
-    int r2, t2;                // 32-row tiles per wave, 32-token tiles per block
+    int nw, t2;                // waves (32 rows each) and 32-token tiles per block
     const uint32_t* fields;
     const uint4* xa;
     MmIn in;
     float* part;
 };
 struct MmTile {
-    int r2, t2, nsplit;
+    int nw, t2, nsplit;
 };
 bool hexmm32_codebook(int n_pts);   // whether launch_hexmm32 covers the codebook
 MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols);

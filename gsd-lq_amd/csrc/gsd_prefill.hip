@@ -62,9 +62,17 @@ __device__ __forceinline__ float mm_finish(const MmSeg& w, const MmIn& in, int m
 // integer fields (r0, r1), exact, from the codebook in LDS; a 64-column
 // block's sum is scaled by its fp16 scale into the fp32 accumulator.
 //
-// A block is 4 waves, each 32 R2 rows, over the same 32 T2 tokens, two
-// blocks per CU.  Bound: the matrix cores and, between them, the latency of
-// the operands.  What the layout is for:
+// A block is NW waves, each 32 rows, over the same 32 T2 tokens, two blocks
+// per CU.  Bound: the matrix cores (32 cycles per product) and, between them,
+// the LDS: 16 code lookups and 8 T2 (high + low) or 4 T2 fragment reads per
+// wave and stage, which follow each other and the products inside a wave.
+// What the layout is for:
+//  * 8 waves where there are rows for them: four waves per SIMD, of which some
+//    read while others multiply, over the same LDS as two.  (4 waves of 64
+//    rows read half the fragments but run two per SIMD: 44-48 % of the matrix
+//    cores' cycles at 512 tokens, with either order of the reads, with raised
+//    priorities, and with the memory's latency taken out.)  923-token prompt
+//    3770 -> 3635 us;
 //  * 32 x 32 tiles: one wave per SIMD issues 1.9 PFLOP/s of them and 1.1 of
 //    16 x 16 tiles (fp16, measured alone), two waves 2.06 against 1.72;
 //  * a lane's half of a 32-row tile comes from lanes (l & 15) + 32 (l >> 5)
@@ -80,22 +88,22 @@ __device__ __forceinline__ float mm_finish(const MmSeg& w, const MmIn& in, int m
 //    waves of a 4-byte LDS read are served in turn, and 28 KB for 217 points
 //    leave room for two blocks per CU.
 // Measured (MI355X, high + low operands, against 16 x 16 tiles with one
-// block per CU): 4096 x 14336 at 512 tokens 143 -> 116 us (1.04 PFLOP/s of
-// matrix-core work), 28672 x 4096 at 512 tokens 311 -> 284 us, at 37 tokens
-// 64 -> 41 us, 6144 x 4096 (q, k and v) at 37 tokens 23 -> 15 us.
+// block per CU): 4096 x 14336 at 512 tokens 143 -> 110 us (1.09 PFLOP/s of
+// matrix-core work), 28672 x 4096 at 512 tokens 311 -> 260 us, at 37 tokens
+// 64 -> 37 us, 6144 x 4096 (q, k and v) at 37 tokens 23 -> 17 us.
 //
 // Safety of the LDS stages.  Stage n goes to buffer n % 3 two stages ahead.
 // A wave waits until only the younger loads than its share of stage n are in
 // flight (vmcnt counts in issue order: the share of stage n + 1, NF loads,
-// and in the second stage of a chunk the 3 R2 code and scale loads issued
+// and in the second stage of a chunk the 3 code and scale loads issued
 // after it) and for its own LDS reads, then meets the others; after that
 // barrier all of stage n is in LDS and no wave reads stage n - 1, whose
 // buffer stage n + 2 then overwrites.
 // ------------------------------------------------------------------------
 constexpr int kMmStages = 3;
-template <int TB, bool HL, int R2, int T2>
-__global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
-    constexpr int NW = 4, TG = 2 * T2, RB = 2 * R2 * NW;   // 16-token groups and 16-row blocks of the block
+template <int TB, bool HL, int T2, int NW>
+__global__ void __launch_bounds__(NW * 64, NW / 2) hexmm32_kernel(const MmArgs a) {
+    constexpr int TG = 2 * T2, RB = 2 * NW;   // 16-token groups and 16-row blocks of the block
     constexpr int NH = HL ? 2 : 1, FPS = 2 * NH;           // fragments of a token group and stage
     constexpr int NF = TG * FPS / NW;                      // fragments (1 KB) a wave moves per stage
     static_assert(NF >= 1 && TG * FPS % NW == 0, "every wave moves whole fragments");
@@ -116,32 +124,24 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
     const int xcd = (bl + 8 - w.x0) & 7, bq = bl >> 3;
     const int rt = (bq / (n_tt * S)) * 8 + xcd, tt = (bq % (n_tt * S)) / S, ks = bq % S;
     if (rt >= n_rt) return;
-    const int rb0 = rt * RB + wid * R2 * 2, g0 = tt * TG;
+    const int rb0 = rt * RB + wid * 2, g0 = tt * TG;
     const int c0 = ks * cps, c1 = min(nc, c0 + cps);
     if (c0 >= c1) return;
     const int half = (lane >> 4) & 1, kg = lane >> 5;
     const uint32_t sh7 = (uint32_t)(lane & 1) * 16u;
 
     // codes and scales of this wave's rows for chunk c
-    const unsigned char* cp[R2];
-    const uint32_t* sp[R2];
-#pragma unroll
-    for (int r = 0; r < R2; r++) {
-        const size_t i = (size_t)min(rb0 + 2 * r + half, nrb - 1) * nc;
-        cp[r] = reinterpret_cast<const unsigned char*>(w.codes_t) + i * TBY + tile_lane_off(B7, (lane & 15) + 32 * kg);
-        sp[r] = w.scales_t + i * 16 + (lane & 15);
-    }
+    const size_t ri = (size_t)min(rb0 + half, nrb - 1) * nc;
+    const unsigned char* cp = reinterpret_cast<const unsigned char*>(w.codes_t) + ri * TBY + tile_lane_off(B7, (lane & 15) + 32 * kg);
+    const uint32_t* sp = w.scales_t + ri * 16 + (lane & 15);
     constexpr int QOFF = B7 ? 28 * 8 : 16 * 16;   // from lane group 2 kg to 2 kg + 1 of a tile
-    u32x4v cw[R2][2];
-    uint32_t sw[R2];
+    u32x4v cw[2];
+    uint32_t sw;
     auto load = [&](int c) {
         c = min(c, nc - 1);
 #pragma unroll
-        for (int r = 0; r < R2; r++) {
-#pragma unroll
-            for (int q = 0; q < 2; q++) cw[r][q] = *reinterpret_cast<const u32x4_a4*>(cp[r] + (size_t)c * TBY + q * QOFF);
-            sw[r] = sp[r][(size_t)c * 16];
-        }
+        for (int q = 0; q < 2; q++) cw[q] = *reinterpret_cast<const u32x4_a4*>(cp + (size_t)c * TBY + q * QOFF);
+        sw = sp[(size_t)c * 16];
     };
     // this wave's fragments of stage 2 c + h (past the end: the last chunk's, unread)
     const u32x4v* ap[NF];
@@ -163,33 +163,15 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
     const uint32_t off = (uint32_t)(lane & 31) * 4u;
     const uint32_t aoff = (uint32_t)(half * FPS * 64 + (lane & 15) + 32 * kg) * 16u;
     uint32_t buf = 0;
-    float16v acc[R2][T2];
+    float16v acc[T2];
 #pragma unroll
-    for (int r = 0; r < R2; r++)
+    for (int g = 0; g < T2; g++)
 #pragma unroll
-        for (int g = 0; g < T2; g++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[r][g][i] = 0.f;
-    uint32_t w4[R2][2][4], sc2[R2];
-    auto look = [&](const uint32_t (&wd)[2][4], auto hc, half8v (&bw)[4]) {
-        constexpr int h = decltype(hc)::value;
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            u32x4v b;
-#pragma unroll
-            for (int e = 0; e < 4; e++) b[e] = *(lds_u32*)(code_addr32<B7>(wd[s >> 1], 8 * h + 4 * (s & 1) + e, off) + TBASE);
-            bw[s] = __builtin_bit_cast(half8v, b);
-        }
-    };
-    auto fold = [&](float16v& ac, const float16v& d, uint32_t s2, auto hc) {
-        constexpr int h = decltype(hc)::value;
-        const float sc = h2f((uint16_t)(h ? (s2 >> 16) : (s2 & 0xFFFFu)));
-#pragma unroll
-        for (int i = 0; i < 16; i++) ac[i] = fmaf(d[i], sc, ac[i]);
-    };
+        for (int i = 0; i < 16; i++) acc[g][i] = 0.f;
+    uint32_t w4[2][4], sc2;
     auto stage = [&](int c, auto hc) {
         constexpr int h = decltype(hc)::value;
-        constexpr int NV = h ? NF + 3 * R2 : NF;   // loads younger than this wave's share of the stage
+        constexpr int NV = h ? NF + 3 : NF;   // loads younger than this wave's share of the stage
         __builtin_amdgcn_s_waitcnt((NV & 15) | ((NV >> 4) << 14) | 0x0F70);
         lds_barrier();
         const uint32_t Ab = buf * ABYTES + aoff;
@@ -200,53 +182,49 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
             load(c + 1);
         }
         __builtin_amdgcn_sched_barrier(0);
-        half8v af[T2][4][NH];
+        half8v af[T2][4][NH], bw[4];
+        auto frags = [&](int hl) {
 #pragma unroll
-        for (int s = 0; s < 4; s++)
+            for (int s = 0; s < 4; s++)
 #pragma unroll
-            for (int g = 0; g < T2; g++)
-#pragma unroll
-                for (int hl = 0; hl < NH; hl++)
+                for (int g = 0; g < T2; g++)
                     af[g][s][hl] = __builtin_bit_cast(half8v, *(lds_u4*)(Ab + (2 * g * FPS + hl * 2 + (s & 1)) * 1024 + 256 * (s >> 1)));
-        // the next rows' operands are decoded, and the last rows' sums
-        // scaled, beside this row tile's products
-        half8v bw[2][4];
-        float16v d[2][T2];
-        look(w4[0], hc, bw[0]);
+        };
+        frags(NH - 1);
 #pragma unroll
-        for (int r = 0; r < R2; r++) {
-            if (r + 1 < R2) look(w4[r + 1], hc, bw[(r + 1) & 1]);
+        for (int s = 0; s < 4; s++) {
+            u32x4v b;
 #pragma unroll
-            for (int g = 0; g < T2; g++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) d[r & 1][g][i] = 0.f;
-            // (low parts first: the block's sum is rounded while it is small)
-#pragma unroll
-            for (int hl = NH - 1; hl >= 0; hl--)
-#pragma unroll
-                for (int s = 0; s < 4; s++)
-#pragma unroll
-                    for (int g = 0; g < T2; g++)
-                        d[r & 1][g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[g][s][hl], bw[r & 1][s], d[r & 1][g], 0, 0, 0);
-            if (r > 0) {
-#pragma unroll
-                for (int g = 0; g < T2; g++) fold(acc[r - 1][g], d[(r - 1) & 1][g], sc2[r - 1], hc);
-            }
+            for (int e = 0; e < 4; e++) b[e] = *(lds_u32*)(code_addr32<B7>(w4[s >> 1], 8 * h + 4 * (s & 1) + e, off) + TBASE);
+            bw[s] = __builtin_bit_cast(half8v, b);
         }
+        if constexpr (HL) frags(0);
+        float16v d[T2];
 #pragma unroll
-        for (int g = 0; g < T2; g++) fold(acc[R2 - 1][g], d[(R2 - 1) & 1][g], sc2[R2 - 1], hc);
+        for (int g = 0; g < T2; g++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) d[g][i] = 0.f;
+        // (low parts first: the block's sum is rounded while it is small)
+#pragma unroll
+        for (int hl = NH - 1; hl >= 0; hl--)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int g = 0; g < T2; g++) d[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[g][s][hl], bw[s], d[g], 0, 0, 0);
+        const float sc = h2f((uint16_t)(h ? (sc2 >> 16) : (sc2 & 0xFFFFu)));
+#pragma unroll
+        for (int g = 0; g < T2; g++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[g][i] = fmaf(d[g][i], sc, acc[g][i]);
     };
     for (int c = c0; c < c1; c++) {
 #pragma unroll
-        for (int r = 0; r < R2; r++) {
+        for (int q = 0; q < 2; q++) {
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) w4[r][q][i] = cw[r][q][i];
-                if constexpr (B7) align7(w4[r][q], sh7);
-            }
-            sc2[r] = sw[r];
+            for (int i = 0; i < 4; i++) w4[q][i] = cw[q][i];
+            if constexpr (B7) align7(w4[q], sh7);
         }
+        sc2 = sw;
         stage(c, std::integral_constant<int, 0>{});
         stage(c, std::integral_constant<int, 1>{});
     }
@@ -254,28 +232,25 @@ __global__ void __launch_bounds__(256, 2) hexmm32_kernel(const MmArgs a) {
     // given back)
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
-    // lane: row l & 31 of each row tile, tokens 8 (i >> 2) + 4 kg + (i & 3)
+    // lane: row l & 31 of the row tile, tokens 8 (i >> 2) + 4 kg + (i & 3)
     float* part = a.part + w.p0;
     const int Mp = ng * 16;
+    const int row = rb0 * 16 + (lane & 31);
+    if (row >= rows) return;
 #pragma unroll
-    for (int r = 0; r < R2; r++) {
-        const int row = (rb0 + 2 * r) * 16 + (lane & 31);
-        if (row >= rows) continue;
+    for (int g = 0; g < T2; g++)
 #pragma unroll
-        for (int g = 0; g < T2; g++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int m = (g0 + 2 * g) * 16 + 8 * (i >> 2) + 4 * kg + (i & 3);
-                if (m >= a.M) continue;
-                if (S > 1) {   // this column split's sum; the consumer adds them in order
-                    part[((size_t)ks * Mp + m) * rows + row] = acc[r][g][i];
-                    continue;
-                }
-                const float y = mm_finish(w, a.in, m, row, acc[r][g][i]);
-                float* yp = w.Y + (size_t)m * rows + row;
-                *yp = a.accumulate ? *yp + y : y;
+        for (int i = 0; i < 16; i++) {
+            const int m = (g0 + 2 * g) * 16 + 8 * (i >> 2) + 4 * kg + (i & 3);
+            if (m >= a.M) continue;
+            if (S > 1) {   // this column split's sum; the consumer adds them in order
+                part[((size_t)ks * Mp + m) * rows + row] = acc[g][i];
+                continue;
             }
-    }
+            const float y = mm_finish(w, a.in, m, row, acc[g][i]);
+            float* yp = w.Y + (size_t)m * rows + row;
+            *yp = a.accumulate ? *yp + y : y;
+        }
 }
 
 // The partial sums of four consecutive rows of token m, in split order
@@ -901,31 +876,31 @@ hipError_t launch_attn_prompt_t(const PrefillAttn& a, dim3 grid, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int TB, bool HL, int R2, int T2>
+template <int TB, bool HL, int T2, int NW>
 hipError_t launch_hexmm32_t(const MmArgs& a, int grid, hipStream_t st) {
     const int lds = kMmStages * 2 * T2 * (HL ? 4 : 2) * 1024 + TB * 128;
     static bool attr = false;
     if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmm32_kernel<TB, HL, R2, T2>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmm32_kernel<TB, HL, T2, NW>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
         attr = true;
     }
-    hipLaunchKernelGGL((hexmm32_kernel<TB, HL, R2, T2>), dim3(grid), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((hexmm32_kernel<TB, HL, T2, NW>), dim3(grid), dim3(NW * 64), lds, st, a);
     return hipGetLastError();
 }
 
 template <int TB>
 hipError_t launch_hexmm32_tb(const MmArgs& a, int grid, hipStream_t st) {
     if (a.hl) {
-        if (a.r2 == 2 && a.t2 == 2) return launch_hexmm32_t<TB, true, 2, 2>(a, grid, st);
-        if (a.r2 == 1 && a.t2 == 2) return launch_hexmm32_t<TB, true, 1, 2>(a, grid, st);
-        if (a.r2 == 1 && a.t2 == 1) return launch_hexmm32_t<TB, true, 1, 1>(a, grid, st);
+        if (a.nw == 8 && a.t2 == 2) return launch_hexmm32_t<TB, true, 2, 8>(a, grid, st);
+        if (a.nw == 4 && a.t2 == 1) return launch_hexmm32_t<TB, true, 1, 4>(a, grid, st);
         return hipErrorInvalidValue;
     }
-    if (a.r2 == 1 && a.t2 == 4) return launch_hexmm32_t<TB, false, 1, 4>(a, grid, st);
-    if (a.r2 == 1 && a.t2 == 2) return launch_hexmm32_t<TB, false, 1, 2>(a, grid, st);
-    if (a.r2 == 1 && a.t2 == 1) return launch_hexmm32_t<TB, false, 1, 1>(a, grid, st);
+    if (a.nw == 8 && a.t2 == 2) return launch_hexmm32_t<TB, false, 2, 8>(a, grid, st);
+    if (a.nw == 4 && a.t2 == 4) return launch_hexmm32_t<TB, false, 4, 4>(a, grid, st);
+    if (a.nw == 4 && a.t2 == 2) return launch_hexmm32_t<TB, false, 2, 4>(a, grid, st);
+    if (a.nw == 4 && a.t2 == 1) return launch_hexmm32_t<TB, false, 1, 4>(a, grid, st);
     return hipErrorInvalidValue;
 }
 
@@ -939,22 +914,25 @@ hipError_t launch_attn_prompt(const PrefillAttn& a, dim3 grid, hipStream_t st) {
 
 bool hexmm32_codebook(int n_pts) { return n_pts == 217 || n_pts == 127; }
 
-// High + low operands (a prompt): two tokens tiles of 32 and two row tiles
-// per wave from 65 tokens on; fewer tokens take narrower tiles, so that the
-// grid is finer and less of a tile is padding.  The columns are split into
+// High + low operands (a prompt): 8 waves over 64 tokens from 33 tokens on (37
+// tokens, 28672 x 4096: 37 us against 41 with 4 waves), 4 over 32 below, where
+// the grid is finer and less of a tile is padding.  The columns are split into
 // what fills two blocks per CU (at least 4 chunks each; up to 16, whose
 // partial sums the next launch still takes in within its own time).
 MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols) {
     const int ng = (M + 15) / 16, nc = (cols + 127) / 128, ncu = device_cu_count() > 0 ? device_cu_count() : 256;
-    MmTile t{ng <= 4 ? 1 : 2, ng <= 2 ? 1 : 2, 1};
-    const int rb = 8 * t.r2, tiles = ((rows_total_tiles_of_16 + rb - 1) / rb) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
+    MmTile t{ng <= 2 ? 4 : 8, ng <= 2 ? 1 : 2, 1};
+    const int rb = 2 * t.nw, tiles = ((rows_total_tiles_of_16 + rb - 1) / rb) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
     t.nsplit = whole_splits(nc, std::max(1, std::min({2 * ncu / tiles, nc / 4, 16})));
     return t;
 }
 
 // Single operands (gsdh_model_matmul), one tensor of a call (tensors of one
-// call tile alike, so a launch may hold several): one row tile per wave and 32, 64 or
-// 128 tokens.  nsplit 0: hexmm_kernel, where the columns would have to be
+// call tile alike, so a launch may hold several): 4 waves over 32 or 64 tokens,
+// from 65 on over 128, which decode a weight least often, or 8 waves over 64
+// where tiles of 128 would hold more padding (with the passes, 8 waves against
+// 4: 28672 x 4096 at 300 tokens 155 and 175 us, 4096 x 14336 96 and 105; at 512
+// 234 and 245, 124 and 122; at 128 92 and 93, 68 and 70).  nsplit 0: hexmm_kernel, where the columns would have to be
 // split and the partial sums' passes (8 bytes per split and output) come to
 // more than about the decode of the weights they spare: measured at 512
 // tokens 4096 x 4096, 37 us there against 31 + 13 here; 4096 x 14336 in four
@@ -962,8 +940,9 @@ MmTile hexmm32_tile_hl(int M, int rows_total_tiles_of_16, int cols) {
 // 48 + 8, 6144 x 4096 at 16 tokens 13 + 4 (three launches of each) against 9 + 3.
 MmTile hexmm32_tile(int M, int rows, int cols) {
     const int ng = (M + 15) / 16, nc = (cols + 127) / 128, ncu = device_cu_count() > 0 ? device_cu_count() : 256;
-    MmTile t{1, ng <= 2 ? 1 : (ng <= 4 ? 2 : 4), 0};
-    const int tiles = ((rows + 127) / 128) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
+    const bool t128 = ng > 4 && (ng + 7) / 8 * 2 == (ng + 3) / 4;
+    MmTile t{ng <= 4 || t128 ? 4 : 8, ng <= 2 ? 1 : (t128 ? 4 : 2), 0};
+    const int tiles = ((rows + 32 * t.nw - 1) / (32 * t.nw)) * ((ng + 2 * t.t2 - 1) / (2 * t.t2));
     const int s = whole_splits(nc, std::max(1, std::min({(nc >= 64 ? 2 * ncu : ncu) / tiles, nc / 4, 16})));
     const bool ok = ng <= 4 || (s == 1 ? 4 * tiles >= 3 * ncu : 32LL * s * ng * 16 <= 5LL * cols);
     t.nsplit = ok && rows % 4 == 0 ? s : 0;
@@ -980,12 +959,12 @@ size_t hexmm32_layout(MmArgs& a, const MmTile& t, int* grid) {
     const int ng = (a.M + 15) / 16, n_tt = (ng + 2 * t.t2 - 1) / (2 * t.t2);
     int b = 0, x = 0;
     size_t p = 0;
-    a.r2 = t.r2;
+    a.nw = t.nw;
     a.t2 = t.t2;
     for (int s = 0; s < a.nseg; s++) {
         MmSeg& w = a.seg[s];
         if (w.nsplit <= 0) w.nsplit = t.nsplit;
-        const int n_rt = ((w.rows + 15) / 16 + 8 * t.r2 - 1) / (8 * t.r2);
+        const int n_rt = ((w.rows + 15) / 16 + 2 * t.nw - 1) / (2 * t.nw);
         w.b0 = b;
         w.x0 = x;
         w.p0 = p;

@@ -82,3 +82,21 @@ def test_any_number_of_prompts(mode, shape):
     assert np.array_equal(first, got)
     assert rel_l2(got, want) < 1e-3
     gpu.close()
+
+
+# 8 waves of 32 rows: 256-row tiles that end inside a wave's rows and with
+# waves past them, more blocks of operands than CUs, the last group of tokens
+# on an XCD of its own round
+@pytest.mark.parametrize("M", [65, 144, 257])
+@pytest.mark.parametrize("name", ["attn_q", "attn_k", "ffn_gate", "ffn_down"])
+def test_matmul_wide_blocks(name, M):
+    banner(f"matmul of {M} tokens, {name}, 8 waves")
+    src, model = _small_model(_spec(n_layers=1, mode="turbo", kinks_per_row=1, **RAGGED))
+    try:
+        key = f"blk.0.{name}.weight"
+        t = dict(src.tensors[key])
+        for f in ("codes", "scales", "row_ptr", "kink_cols", "kink_deltas"):
+            t[f] = np.ascontiguousarray(src.hex_field(key, f))
+        check(model, t, 0, SLOTS[name], M, seed=M + SLOTS[name])
+    finally:
+        model.close()
