@@ -36,9 +36,12 @@ __device__ __forceinline__ uint32_t code_addr32(const uint32_t (&w)[4], int j, u
 
 // 64 lanes x 16 bytes from global memory into LDS at byte lds + 16 * lane,
 // past the registers (no output register, so nothing is allocated to the
-// load in flight; the caller waits on vmcnt before any wave reads the bytes)
+// load in flight; the caller waits on vmcnt before any wave reads the bytes).
+// A scalar write of m0 needs one wait state before a load to LDS reads it, and
+// the compiler adds none inside an asm block: without the s_nop the load could
+// take the last m0 and put its 1 KB there.
 __device__ __forceinline__ void lds_dma16(const void* p, uint32_t lds) {
-    __asm__ volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
 }
 
 // y of one (token, row): the descaled sum s, kinks, rank-k
