@@ -671,11 +671,12 @@ int issue_ffn(gsdh_model* m, int l, bool with_o) {
     return 0;
 }
 
-int issue_linear(gsdh_model* m, int l, int mask) {
+int issue_linear(gsdh_model* m, int l, int mask, bool fuse = true) {
     int rc = 0;
     // gate/up and down together: one fused FFN launch where it covers the
-    // layer, with o in it too where o is issued with them
-    const bool fffn = (mask & 12) == 12 && ffn_fused(m, l);
+    // layer (and the caller lets it), with o in it too where o is issued with
+    // them
+    const bool fffn = fuse && (mask & 12) == 12 && ffn_fused(m, l);
     const bool fo = fffn && (mask & 2) && offn_fused(m, l);
     if (mask & 1) {
         HexArgs a = qkv_args(m, l);
@@ -1004,8 +1005,12 @@ int issue_prefill(gsdh_model* m, int M, int p0) {
     return 0;
 }
 
-// One decode layer without the fused attention: the step's q/k/v, attention
-// and o + FFN launches for x at the step position.
+// One decode layer for x at the step position, a launch per projection.  No
+// block of it waits for one that may not have started: the fused o + FFN
+// launch needs all its blocks resident at once, and those of two models'
+// prompts on two threads can hold each other's places until both give up.
+// (37-token turn of the 7B shape, two layers: 274 us with the fused launch,
+// 283 so.)
 int issue_layer(gsdh_model* m, int l) {
     const auto& c = m->c;
     int rc = issue_linear(m, l, 1);
@@ -1018,7 +1023,7 @@ int issue_layer(gsdh_model* m, int l) {
         HIPCHK(launch_rope_kv(m->q, m->k, m->v, r, nullptr, m->stream));
     }
     HIPCHK(launch_attention(layer_attention(m, l, 0), m->stream));
-    return issue_linear(m, l, 2 | 4 | 8);
+    return issue_linear(m, l, 2 | 4 | 8, false);
 }
 
 // Prompt tokens P.tok[0..M) at positions p0.. on the 32 x 32 tile
