@@ -4,11 +4,17 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gsd_lds_limit.h"
+
 namespace gsd {
 
 constexpr int kMaxSeg = 3;        // q, k, v share one launch
 constexpr int kMaxRank = 16;      // tmp_k scratch of the reference is 16 floats
 constexpr int kTableSlots = 256;  // LDS codebook slots (codes are u8)
+
+inline hipError_t raise_lds_limit(LdsLimit& limit, const void* kernel, size_t lds) {
+    return limit.raise(lds, [&](size_t n) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n); });
+}
 
 // One packed tensor of a fused matvec launch.  All pointers are device
 // pointers in the .gsd2 field layout (codes row-major u8 pairs, fp16 scales

@@ -3258,20 +3258,13 @@ static bool half_units_reach(const HexArgs& a) {
 
 template <int TB, int LR, int EPI, int DEP = kMv4Depth>
 hipError_t launch_hexmv4_t(const HexArgs& a0, hipStream_t st, int nw, size_t lds, int nunits, int nlead) {
-    static int per_cu = 0;
-    static size_t attr_lds = 0;
-    if (lds > attr_lds) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmv4_kernel<TB, LR, EPI, 0, 0, DEP>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr_lds = lds;
-        per_cu = 0;
-    }
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, hexmv4_kernel<TB, LR, EPI, 0, 0, DEP>, nw * 64, lds) != hipSuccess ||
-        n < 1)
+    static LdsLimit limit;
+    const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&hexmv4_kernel<TB, LR, EPI, 0, 0, DEP>), lds);
+    if (e != hipSuccess) return e;
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, hexmv4_kernel<TB, LR, EPI, 0, 0, DEP>, nw * 64, lds) != hipSuccess ||
+        per_cu < 1)
         return hipErrorInvalidConfiguration;
-    per_cu = n;
     const int ncu = device_cu_count() > 0 ? device_cu_count() : 256;
     // publishing blocks (LR == 2) first (dispatched in order, they are
     // resident before any matvec block waits on them), and all blocks
@@ -3309,13 +3302,10 @@ hipError_t launch_hexmv4_t(const HexArgs& a0, hipStream_t st, int nw, size_t lds
 template <int TB, int LR, int HD, int G, int PW>
 hipError_t launch_qkva_t(const HexArgs& a0, hipStream_t st, int nw, size_t lds, int nunits) {
     const int nt = (nw > 8 ? nw : 8) * 64;
-    static size_t attr_lds = 0;
-    if (lds > attr_lds) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmv4_kernel<TB, LR, kEpiRopeKV, HD, G, kMv4Depth, PW>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr_lds = lds;
-    }
+    static LdsLimit limit;
+    const hipError_t e =
+        raise_lds_limit(limit, reinterpret_cast<const void*>(&hexmv4_kernel<TB, LR, kEpiRopeKV, HD, G, kMv4Depth, PW>), lds);
+    if (e != hipSuccess) return e;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, hexmv4_kernel<TB, LR, kEpiRopeKV, HD, G, kMv4Depth, PW>, nt, lds) != hipSuccess || per_cu < 1)
         return hipErrorNotSupported;
@@ -3464,13 +3454,9 @@ hipError_t launch_hexmm_t(const MatmulArgs& a, hipStream_t st) {
     const int grid = 8 * n_tt * a.nsplit * ((n_rt + 7) / 8);
     const size_t lds = TB > 0 ? 0 : (size_t)a.w.n_pts * 256;
     if (lds > 0) {
-        static size_t attr = 0;
-        if (lds > attr) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmm_kernel<TB, TG, RBW, HL>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            attr = lds;
-        }
+        static LdsLimit limit;
+        const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&hexmm_kernel<TB, TG, RBW, HL>), lds);
+        if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL((hexmm_kernel<TB, TG, RBW, HL>), dim3(grid), dim3(512), lds, st, a);
     hipError_t e = hipGetLastError();
@@ -3554,13 +3540,9 @@ hipError_t launch_batch_prep(const BatchPrep& p, hipStream_t st) {
     for (int g = 0; g < kMaxSeg; g++) fast = fast && p.k[g] <= 2 && (p.k[g] == 0 || (reinterpret_cast<uintptr_t>(p.Vt[g]) & 7) == 0);
     if (fast) {
         const size_t lds = (size_t)p.cols * 4;
-        static size_t attr = 0;
-        if (lds > attr) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&batch_prep2_kernel),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            attr = lds;
-        }
+        static LdsLimit limit;
+        const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&batch_prep2_kernel), lds);
+        if (e != hipSuccess) return e;
         hipLaunchKernelGGL(batch_prep2_kernel, dim3(((p.M + 15) / 16) * 16), dim3(512), lds, st, p);
         return hipGetLastError();
     }

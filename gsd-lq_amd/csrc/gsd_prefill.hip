@@ -868,13 +868,9 @@ template <int HD>
 hipError_t launch_attn_prompt_t(const PrefillAttn& a, dim3 grid, hipStream_t st) {
     constexpr int lds = 4 * 2 * (32 * (HD + 8) * 2 + HD * 36 * 2);
     static_assert(lds >= 2048 + 2 * 4 * (HD / 32) * 4 * 64 * 16 && lds <= 160 * 1024, "the merge fits the stages");
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prompt_kernel<HD>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static LdsLimit limit;
+    const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&attn_prompt_kernel<HD>), lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((attn_prompt_kernel<HD>), grid, dim3(512), lds, st, a);
     return hipGetLastError();
 }
@@ -882,13 +878,9 @@ hipError_t launch_attn_prompt_t(const PrefillAttn& a, dim3 grid, hipStream_t st)
 template <int TB, bool HL, int T2, int NW>
 hipError_t launch_hexmm32_t(const MmArgs& a, int grid, hipStream_t st) {
     const int lds = kMmStages * 2 * T2 * (HL ? 4 : 2) * 1024 + TB * 128;
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hexmm32_kernel<TB, HL, T2, NW>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static LdsLimit limit;
+    const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&hexmm32_kernel<TB, HL, T2, NW>), lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((hexmm32_kernel<TB, HL, T2, NW>), dim3(grid), dim3(NW * 64), lds, st, a);
     return hipGetLastError();
 }
@@ -1028,13 +1020,9 @@ hipError_t launch_layer_prep(const LayerPrep& p, LayerPrepIn in, hipStream_t st)
     const bool wide = (int)grid.x <= (device_cu_count() > 0 ? device_cu_count() : 256);
 #define GSD_PREP_N(IN, NT)                                                                                               \
     {                                                                                                                    \
-        static size_t attr = 0;                                                                                          \
-        if (lds > attr) {                                                                                                \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&layer_prep_kernel<IN, NT>),          \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);              \
-            if (e != hipSuccess) return e;                                                                               \
-            attr = lds;                                                                                                  \
-        }                                                                                                                \
+        static LdsLimit limit;                                                                                           \
+        const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&layer_prep_kernel<IN, NT>), lds);     \
+        if (e != hipSuccess) return e;                                                                                   \
         hipLaunchKernelGGL((layer_prep_kernel<IN, NT>), grid, dim3(NT), lds, st, p);                                     \
     }
 #define GSD_PREP(IN) if (wide) GSD_PREP_N(IN, 1024) else GSD_PREP_N(IN, 512) break;
