@@ -800,15 +800,26 @@ hipGraphExec_t step_graph(const gsdh_model* m, int pos) {
 
 // Staging bytes of one gsdh_model_matmul call (bf16 X, single fp16 operand
 // rounding): A fragments, descales, rank-k values (one slot per tensor of a
-// shared-input call), split partials.
-size_t matmul_ws_need(int M, int rows, int cols) {
+// shared-input call), then the split partials.
+size_t matmul_operand_bytes(int M, int cols) {
     const size_t xa = (hexmm_xa_bytes(M, cols) + 255) / 256 * 256;
     const size_t xs = ((size_t)(M + 15) / 16 * 16 * 4 + 255) / 256 * 256;
     const size_t tk = ((size_t)M * kMaxRank * 4 + 255) / 256 * 256;
+    return xa + xs + kMaxSeg * tk;
+}
+
+// Split partials of one tensor on the 32 x 32 tiles (0: not split, or not on them)
+size_t matmul32_part_bytes(int M, int rows, int cols) {
+    const MmTile t = hexmm32_tile(M, rows, cols);
+    return t.nsplit > 1 ? (size_t)t.nsplit * ((M + 15) / 16 * 16) * rows * 4 : 0;
+}
+
+// with the partials of either path (the 16 x 16 tiles serve a Y that is not
+// 16-byte aligned)
+size_t matmul_ws_need(int M, int rows, int cols) {
     const MatmulPlan plan = hexmm_plan(M, rows, cols);
-    const MmTile t = hexmm32_tile(M, rows, cols);   // (its launch holds up to kMaxSeg tensors' partial sums)
-    const size_t n = std::max(plan.nsplit > 1 ? plan.nsplit : 0, t.nsplit > 1 ? kMaxSeg * t.nsplit : 0);
-    return xa + xs + kMaxSeg * tk + n * ((M + 15) / 16 * 16) * rows * 4;
+    const size_t pt = plan.nsplit > 1 ? (size_t)plan.nsplit * ((M + 15) / 16 * 16) * rows * 4 : 0;
+    return matmul_operand_bytes(M, cols) + std::max(pt, matmul32_part_bytes(M, rows, cols));
 }
 
 size_t split_part_bytes(int M, int rows, int cols) {   // the prefill's (high + low operands)
@@ -878,6 +889,11 @@ int setup_batched(gsdh_model* m) {
             if (M <= kPrefillChunk) part = std::max(part, split_part_bytes(M, sh[0], sh[1]));
         }
         mm = std::max(mm, matmul_ws_need(M, c.vocab, c.hidden));
+        // one launch's partials of the tensors that a layer reads one input
+        // with (other sets that do not fit together take a launch each)
+        mm = std::max(mm, matmul_operand_bytes(M, c.hidden) +
+                              std::max(matmul32_part_bytes(M, qd, c.hidden) + 2 * matmul32_part_bytes(M, kvd, c.hidden),
+                                       2 * matmul32_part_bytes(M, c.ffn, c.hidden)));
         if (M <= kPrefillChunk && M % 16 == 0) part = std::max(part, prompt_part_bytes(m, M));
     }
     auto& P = m->pf;
@@ -897,13 +913,17 @@ int setup_batched(gsdh_model* m) {
     A((void**)&P.A, (size_t)Mc * qd * 4);
     A((void**)&P.G, (size_t)Mc * c.ffn * 4);
     A((void**)&P.U, (size_t)Mc * c.ffn * 4);
-    A((void**)&P.xn, (size_t)Mp * maxc * 4);
+    // the prepared input in fp32: the kink terms' (and batch_prep_kernel's)
+    const bool mm32 = prompt_mm32(m);
+    bool kinks = false;
+    for (const HexDev& t : m->hex) kinks = kinks || t.nk > 0;
+    if (!mm32 || kinks) A((void**)&P.xn, (size_t)Mp * maxc * 4);
     A((void**)&P.xa, hexmm_xa_bytes(Mc, maxc, 1));
     A((void**)&P.xs, (size_t)Mp * 4);
     A((void**)&P.tmp, (size_t)kMaxSeg * Mc * kMaxRank * 4);
     A((void**)&P.part, part);
-    if (prompt_mm32(m)) {
-        A((void**)&P.xn1, (size_t)Mp * maxc * 4);
+    if (mm32) {
+        if (kinks) A((void**)&P.xn1, (size_t)Mp * maxc * 4);
         A((void**)&P.xs1, (size_t)Mp * 4);
         A((void**)&P.tmp1, (size_t)kMaxSeg * Mc * kMaxRank * 4);
     }
@@ -1625,7 +1645,9 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
     float* xsp = reinterpret_cast<float*>(w + xa);
     // (split partials of the tensors in turn, or of one launch's tensors
     // after each other: stream order keeps the calls apart)
-    float* part = reinterpret_cast<float*>(w + xa + xs + kMaxSeg * tk);
+    float* part = reinterpret_cast<float*>(w + matmul_operand_bytes(M, cols));
+    const size_t part_bytes = m->mm_ws_bytes - matmul_operand_bytes(M, cols);
+    size_t part_used = 0;   // by the tensors of the launch that is being put together
     // X's operands once for every tensor of the call, with the rank-k
     // products where one pass covers them
     MmXprep xp{};
@@ -1655,6 +1677,7 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
         HIPCHK(launch_hexmm32(a, grid, m->stream));
         HIPCHK(launch_mm_reduce(a, m->stream));
         a.nseg = 0;
+        part_used = 0;
         return 0;
     };
     int rc = 0;
@@ -1664,7 +1687,9 @@ int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, 
         const MmTile tile = hexmm32_codebook(n_pts) && (reinterpret_cast<uintptr_t>(Y[i]) & 15) == 0 ? hexmm32_tile(M, t.rows, cols)
                                                                                                     : MmTile{};
         if (tile.nsplit > 0) {
-            if (a.nseg && a.n_pts != n_pts && (rc = flush())) return rc;
+            const size_t need = matmul32_part_bytes(M, t.rows, cols);
+            if (a.nseg && (a.n_pts != n_pts || part_used + need > part_bytes) && (rc = flush())) return rc;
+            part_used += need;
             a.n_pts = n_pts; a.fields = m->fields[t.radius]; a.nw = tile.nw; a.t2 = tile.t2;
             MmSeg& sg = a.seg[a.nseg++];
             sg = mm_seg(t, Y[i]);

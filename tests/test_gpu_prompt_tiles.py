@@ -5,13 +5,15 @@ oracle: token counts at the edges of 16-token groups and of the 32- and
 tiles, columns that end in half a chunk and columns whose chunks do not divide
 into the splits, both code formats, kinks and rank-2 terms taken in from
 column splits; and that a model takes any number of prompts."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle as O
 from conftest import rel_l2
-from gpu_util import banner
-from test_gpu_prefill import SLOTS, _kv_close, _pair, _small_model, _spec, check
+from gpu_util import D, E, H, banner
+from test_gpu_prefill import SLOTS, _kv_close, _pair, _small_model, _spec, bf16, check, layer_shape, run_matmul, turbo_7b  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +102,44 @@ def test_matmul_wide_blocks(name, M):
         check(model, t, 0, SLOTS[name], M, seed=M + SLOTS[name])
     finally:
         model.close()
+
+
+def _shared(model, names, xb, M, rows):
+    lib = model.cl.lib
+    dx, ys = D(xb), [E(M * r * 4) for r in rows]
+    slots = (ctypes.c_int * len(names))(*[SLOTS[n] for n in names])
+    lib.gsdh_model_matmul_shared(model._m, 0, slots, len(names), dx.ptr, M,
+                                 (ctypes.c_void_p * len(names))(*[y.ptr.value for y in ys]))
+    lib.gsdh_stream_sync(lib.gsdh_model_stream(model._m))
+    return [H(y, np.float32, M * r).reshape(M, r) for y, r in zip(ys, rows)]
+
+
+# sets whose partial sums fit the workspace together, and sets that take a
+# launch for each tensor or two: any tensors of equal columns share a call
+@pytest.mark.parametrize("names,M", [(("ffn_down",) * 3, 512), (("ffn_gate", "attn_q", "ffn_up"), 128),
+                                     (("ffn_gate",) * 3, 128), (("attn_output", "attn_q", "attn_q"), 64)])
+def test_matmul_any_set_equals_separate_calls(turbo_7b, names, M):  # noqa: F811
+    banner(f"shared-input matmul {names} M={M}")
+    _, model = turbo_7b
+    rows = [layer_shape(n)[0] for n in names]
+    xb, _ = bf16(np.random.default_rng(M).standard_normal((M, layer_shape(names[0])[1])).astype(np.float32))
+    want = {n: run_matmul(model, 0, SLOTS[n], xb, M, r) for n, r in zip(names, rows)}
+    for n, got in zip(names, _shared(model, names, xb, M, rows)):
+        assert np.array_equal(got, want[n]), n
+
+
+def test_model_memory(turbo_7b):  # noqa: F811
+    """A model's memory beyond its tensors, embedding and cache: the partial
+    sums of the largest set of tensors that share an input (33.5 MB, down at 512
+    tokens), and no copy of the inputs for kink terms that it does not have."""
+    _, model = turbo_7b
+    packed = sum(r * c // 2 + r * c // 32 for r, c in [layer_shape(n) for n in SLOTS] + [(32768, 4096)])
+    slabs = 4096 * 14336 // 2 + 4096 * 14336 // 32       # down again, for the fused launch
+    embedding, cache = 2 * 32768 * 4096, 4 * 640 * 1024
+    rest = model.cl.allocated_bytes - packed - slabs - embedding - cache
+    tokens = 512
+    prompt = 4 * tokens * (2 * 4096 + 2 * 1024 + 4096 + 2 * 14336) + 8 * tokens * 14336
+    operands, parts = 4 * tokens * 14336, 4 * 4 * tokens * 4096
+    print(f"[gpu-test] beyond tensors, embedding and cache: {rest / 1e6:.1f} MB "
+          f"({(rest - prompt - operands - parts) / 1e6:.1f} above the prompt's rows, the operands and one set's sums)", flush=True)
+    assert rest - prompt - operands - parts < 20e6       # (the prompts' own partial sums, decode's hand-off words)
