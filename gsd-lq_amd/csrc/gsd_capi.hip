@@ -1727,6 +1727,14 @@ int gsdh_matmul_plan(int M, int rows, int cols, int* tg, int* rbw, int* nsplit) 
     return 0;
 }
 
+int gsdh_matmul_tile(int M, int rows, int cols, int n_pts, int* waves, int* tokens) {
+    if (M <= 0 || rows <= 0 || cols <= 0 || !waves || !tokens) return fail(-1, "matmul_tile: bad argument");
+    const MmTile t = hexmm32_codebook(n_pts) ? hexmm32_tile(M, rows, cols) : MmTile{};
+    *waves = t.nsplit > 0 ? t.nw : 0;
+    *tokens = t.nsplit > 0 ? 32 * t.t2 : 0;
+    return 0;
+}
+
 int gsdh_model_run_linear(gsdh_model* m, int layer, int mask) {
     if (!m) return fail(-1, "run_linear: null model");
     if (mask & ~31) return fail(-1, "run_linear: mask 0x%x", mask);

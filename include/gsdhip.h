@@ -293,12 +293,17 @@ int gsdh_model_matmul(gsdh_model* m, int layer, int slot, const uint16_t* X, int
  * calls, bit for bit. */
 int gsdh_model_matmul_shared(gsdh_model* m, int layer, const int* slots, int n, const uint16_t* X, int M,
                              float* const* Y);
-/* The tiling gsdh_model_matmul and the batched prefill use for M tokens of a
- * rows x cols tensor on the current device: token groups of 16 per block
- * (*tg: 1, 2, 4, 8), row blocks of 16 per wave (*rbw) and column splits
- * (*nsplit).  A diagnostic (tests name the tiles they run); no reference
- * counterpart. */
+/* The tiling gsdh_model_matmul uses for M tokens of a rows x cols tensor on the
+ * current device: token groups of 16 per block (*tg), row blocks of 16 per wave
+ * (*rbw) and column splits (*nsplit); of the 32 x 32 tile kernel where it takes
+ * the shape (codebooks of 127 or 217 points), else of the 16 x 16 one.  (A
+ * prompt's projections are tiled by rules of their own.)  A diagnostic (tests
+ * name the tiles they run); no reference counterpart. */
 int gsdh_matmul_plan(int M, int rows, int cols, int* tg, int* rbw, int* nsplit);
+/* The 32 x 32 tile kernel's block for that call and a codebook of n_pts points:
+ * waves of 32 rows (4 or 8) and tokens (32, 64 or 128), or 0 and 0 where the
+ * 16 x 16 tiles run.  A diagnostic; no reference counterpart. */
+int gsdh_matmul_tile(int M, int rows, int cols, int n_pts, int* waves, int* tokens);
 
 /* The codes of packed tensor (layer, slot) as the device holds them, decoded
  * back to the file's u8 [rows][cols/2] order on the device by the same tile

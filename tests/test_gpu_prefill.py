@@ -157,18 +157,14 @@ def layer_shape(name):
 
 
 def test_prefill_7b_turbo_chunks(turbo_7b):
-    """The batched prefill forward of the 7B Turbo layer (32 / 8 heads of
-    128, ffn 14336, vocab 32768): 514 tokens (a 512-token chunk: eight-group
-    tiles with two row blocks per wave; then a 2-token chunk on column-split
-    tiles), then 64 more after that prefix (two-group tiles), against the
-    oracle's token-by-token forward."""
+    """The batched prefill forward of one 7B Turbo layer (32 / 8 heads of 128,
+    ffn 14336, vocab 32768): 514 tokens (chunks of 512 and 2), then 64 more
+    after that prefix, against the oracle's token-by-token forward.  One layer
+    is the last one: K and V of every token, the rest of the last token as a
+    decode step."""
     import bench
     bank, model = turbo_7b
     banner("batched prefill 7B turbo: 514 tokens, then 64 more")
-    lib = model.cl.lib
-    for M in (512, 2, 64):
-        print(f"[gpu-test] chunk {M}: gate/up plan {plan(lib, M, 14336, 4096)}, q plan {plan(lib, M, 4096, 4096)}, "
-              f"down plan {plan(lib, M, 4096, 14336)}", flush=True)
     ref = O.OracleModel(bench.BankSource(bank, 1), kind="port", max_seq_len=640, rope_interleaved=1)
     toks = np.random.default_rng(130).integers(0, model.vocab_size, 578).tolist()
     got = model.prefill(toks[:514], 0)
