@@ -400,3 +400,36 @@ def test_greedy_argmax_special_values(lib, name, split):
         assert int(H(tok, np.int32, 1)[0]) == want, (name, call)
         assert H(mg, np.float32, 1)[0] == want_margin, (name, call)
     assert np.all(H(ctr, np.uint32) == 2), name
+
+
+# columns of several rounds per wave (and the most there are), rows that end
+# inside a block, more kinks in a row than lanes, rows without any beside them
+@pytest.mark.parametrize("rows,cols,R,k,per", [(9, 65536, 8, 0, (0, 3)), (17, 4160, 6, 2, (150, 0, 1)), (8, 1088, 6, 1, (65, 64))])
+def test_hex2d_matvec_uneven_kinks(lib, rows, cols, R, k, per):
+    banner(f"matvec {rows}x{cols} R{R} k{k}, kinks {per} in turn")
+    f = dict(_pack(rows, cols, R, k, 0))
+    rng = np.random.default_rng(rows)
+    n = [per[r % len(per)] for r in range(rows)]
+    f["row_ptr"] = np.concatenate([[0], np.cumsum(n)]).astype(np.uint32)
+    f["kink_cols"] = np.concatenate([np.sort(rng.choice(cols, m, replace=False)) for m in n]).astype(np.uint16)
+    f["kink_deltas"] = (0.06 * rng.standard_normal(sum(n))).astype(np.float32)
+    x = rng.standard_normal(cols).astype(np.float32)
+    tk = rng.standard_normal(k).astype(np.float32) if k else None
+    assert rel_l2(_gpu_matvec(lib, f, x, tk), O.hex2d_matvec(x, f, tmp_k=tk)) < 1e-5   # fp32 accumulation order only
+
+
+# wide loads where columns and pointers let them, single ones elsewhere
+@pytest.mark.parametrize("cols,x_off,v_off", [(4096, 0, 0), (4100, 0, 0), (16388, 0, 0), (4, 0, 0), (4098, 0, 0), (1, 0, 0),
+                                              (1023, 0, 0), (4096, 4, 0), (4096, 0, 2), (4096, 0, 4)])
+def test_lowrank_routes(lib, cols, x_off, v_off, k=3):
+    banner(f"rank projection, {cols} columns, x off by {x_off}, Vt by {v_off} bytes")
+    rng = np.random.default_rng(cols)
+    x, S = rng.standard_normal(cols).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    Vt = rng.standard_normal((k, cols)).astype(np.float16)
+    dx = D(np.concatenate([np.zeros(x_off // 4, np.float32), x]))
+    dv, ds, tk = D(np.concatenate([np.zeros(v_off // 2, np.float16), Vt.reshape(-1)])), D(S), E(64)
+    lib.gsdh_lowrank_proj(None, dx.ptr.value + x_off, dv.ptr.value + v_off, p(ds), p(tk), k, cols)
+    want = S.astype(np.float64) * (Vt.astype(np.float64) @ x.astype(np.float64))
+    scale = np.abs(S) * (np.abs(Vt.astype(np.float64)) @ np.abs(x.astype(np.float64)))
+    # fp32 sums of 1024 threads' chains: an error of each addition, 2^-24 of what is added up
+    assert (np.abs(H(tk, np.float32, k) - want) <= 2.0 ** -24 * (cols / 1024 + 16) * scale).all()
