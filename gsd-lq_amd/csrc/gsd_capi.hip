@@ -50,21 +50,9 @@ namespace {
 
 inline hipStream_t S(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
-// Codebook of radius R as float2 (gsd_lq_cpu_runtime.py:111-118).
-std::vector<float> host_table(int R) {
-    std::vector<float> t;
-    const double s32 = std::sqrt(3.0) / 2.0;
-    for (int a = -R; a <= R; a++)
-        for (int b = -R; b <= R; b++) {
-            if (std::abs(a + b) > R) continue;
-            t.push_back((float)((double)a + 0.5 * (double)b));
-            t.push_back((float)((double)b * s32));
-        }
-    return t;
-}
-
 // Integer fields (r0, r1) of the radius-R codewords in enumeration order, as
-// fp16 pairs (low half r0): the lattice form of the same table.
+// fp16 pairs (low half r0): the lattice form of the codebook
+// (gsd_lq_cpu_runtime.py:111-118).
 uint16_t half_of_small_int(int n) {
     if (n == 0) return 0;
     const uint16_t sign = n < 0 ? 0x8000u : 0u;
@@ -461,7 +449,6 @@ struct HexDev {
 struct gsdh_model {
     gsdh_model_config c{};
     hipStream_t stream = nullptr;
-    float* tables[9] = {};          // by radius: codeword points
     uint32_t* fields[9] = {};       // by radius: (r0, r1) fp16 pairs
     uint16_t* embed = nullptr;
     float* norms = nullptr;         // [n_layers][2][hidden] + output [hidden]
@@ -550,7 +537,7 @@ int dalloc(gsdh_model* m, void** p, size_t n) {
 void fill_seg(HexSeg& s, const HexDev& t, const gsdh_model* m, float* out) {
     s.codes_t = t.codes_t; s.scales_t = t.scales_t; s.row_ptr = t.nk ? t.row_ptr : nullptr;
     s.kcols = t.kcols; s.kdel = t.kdel; s.U = t.U; s.Vt = t.Vt; s.S = t.Sv; s.tmp_k = nullptr;
-    s.table = m->tables[t.radius]; s.fields = m->fields[t.radius]; s.out = out; s.rows = t.rows; s.k = t.k;
+    s.fields = m->fields[t.radius]; s.out = out; s.rows = t.rows; s.k = t.k;
     s.n_pts = 3 * t.radius * t.radius + 3 * t.radius + 1;
 }
 
@@ -578,7 +565,6 @@ HexArgs qkv_args(gsdh_model* m, int l) {
     fill_seg(a.seg[1], m->slot(l, GSDH_K), m, m->k);
     fill_seg(a.seg[2], m->slot(l, GSDH_V), m, m->v);
     a.x = m->x; a.norm_w = m->norm(l, 0); a.eps = c.rms_eps; a.cols = c.hidden; a.epilogue = kEpiStore;
-    a.scale_t = 1;
     if (c.rope_interleaved) {
         a.epilogue = kEpiRopeKV;
         RopeKV& r = a.rope;
@@ -689,7 +675,6 @@ int issue_linear(gsdh_model* m, int l, int mask, bool fuse = true) {
         a.nseg = 1;
         fill_seg(a.seg[0], m->slot(l, GSDH_O), m, m->x);
         a.x = m->attn; a.cols = c.n_heads * c.head_dim; a.epilogue = kEpiResidual; a.resid = m->x;
-        a.scale_t = 1;
         if ((rc = prep_lowrank(m, a))) return rc;
         HIPCHK(launch_hexmv4(a, m->stream));
     }
@@ -700,7 +685,6 @@ int issue_linear(gsdh_model* m, int l, int mask, bool fuse = true) {
         fill_seg(a.seg[0], m->slot(l, GSDH_GATE), m, m->h);
         fill_seg(a.seg[1], m->slot(l, GSDH_UP), m, nullptr);
         a.x = m->x; a.norm_w = m->norm(l, 1); a.eps = c.rms_eps; a.cols = c.hidden; a.epilogue = kEpiSwiGLU;
-        a.scale_t = 1;
         if ((rc = prep_lowrank(m, a))) return rc;
         HIPCHK(launch_hexmv4(a, m->stream));
     }
@@ -709,7 +693,6 @@ int issue_linear(gsdh_model* m, int l, int mask, bool fuse = true) {
         a.nseg = 1;
         fill_seg(a.seg[0], m->slot(l, GSDH_DOWN), m, m->x);
         a.x = m->h; a.cols = c.ffn; a.epilogue = kEpiResidual; a.resid = m->x;
-        a.scale_t = 1;
         if ((rc = prep_lowrank(m, a))) return rc;
         HIPCHK(launch_hexmv4(a, m->stream));
     }
@@ -725,7 +708,6 @@ int issue_head(gsdh_model* m, bool greedy, bool to_host = false) {
     a.nseg = 1;
     fill_seg(a.seg[0], m->slot(0, GSDH_LM_HEAD), m, m->logits);
     a.x = m->x; a.norm_w = m->norm(-1, 0); a.eps = c.rms_eps; a.cols = c.hidden; a.epilogue = kEpiStore;
-    a.scale_t = 1;
     int rc = prep_lowrank(m, a);
     if (rc) return rc;
     HIPCHK(launch_hexmv4(a, m->stream));
@@ -1244,12 +1226,6 @@ int gsdh_model_create(const gsdh_model_config* cfg, gsdh_model** out) {
     A((void**)&m->gen_tok, (size_t)c.max_seq_len * 4);
     A((void**)&m->gen_margin, (size_t)c.max_seq_len * 4);
     for (int R = 1; R <= 8; R++) {
-        std::vector<float> t = host_table(R);
-        A((void**)&m->tables[R], t.size() * 4);
-        if (!rc) {
-            e = hipMemcpy(m->tables[R], t.data(), t.size() * 4, hipMemcpyHostToDevice);
-            if (e != hipSuccess) rc = fail((int)e, "hipMemcpy table: %s", hipGetErrorString(e));
-        }
         std::vector<uint32_t> f = host_fields(R);
         f.resize(kTableSlots, 0u);   // padded: the matvec reads 16-entry slices
         A((void**)&m->fields[R], f.size() * 4);

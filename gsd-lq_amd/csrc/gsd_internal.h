@@ -17,11 +17,9 @@ inline hipError_t raise_lds_limit(LdsLimit& limit, const void* kernel, size_t ld
 }
 
 // One packed tensor of a fused matvec launch.  All pointers are device
-// pointers in the .gsd2 field layout (codes row-major u8 pairs, fp16 scales
-// per 64 weights, CSR kinks, U [rows,k], Vt [k,cols]).
+// pointers: codes and scales in the tiled layout below, the rest in the .gsd2
+// field layout (CSR kinks, U [rows,k], Vt [k,cols]).
 struct HexSeg {
-    const uint8_t* codes;
-    const uint16_t* scales;
     const uint32_t* row_ptr;   // null: no kinks
     const uint16_t* kcols;
     const float* kdel;
@@ -29,10 +27,8 @@ struct HexSeg {
     const uint16_t* Vt;        // k > 0 and tmp_k == null: computed in-kernel
     const float* S;
     const float* tmp_k;        // k > 0: precomputed low-rank projection, or null
-    const float* table;        // float2 [n_pts]: codeword points (generic path)
     // half2 [n_pts] integer fields (r0, r1) of the A2 codewords, whose points
-    // are (r0 + r1/2, r1*sqrt(3)/2); non-null in every segment selects the
-    // lattice path (requires scale_t = 1)
+    // are (r0 + r1/2, r1*sqrt(3)/2)
     const uint32_t* fields;
     // tiled device layout of the MFMA path (hexmv4):
     //   codes_t  [ceil(rows/16)][ceil(cols/128)][64 lanes][16 B]
@@ -44,7 +40,7 @@ struct HexSeg {
     const uint4* codes_t;
     const uint32_t* scales_t;
     float* out;
-    int rows, k, n_pts, batch0;
+    int rows, k, n_pts;
 };
 
 enum HexEpilogue : int {
@@ -72,10 +68,7 @@ struct HexArgs {
     float eps;
     float* resid;          // kEpiResidual target (read-modify-write)
     int cols;
-    int nbatch;            // row batches in total
     int epilogue;
-    int scale_t;           // scales layout: 0 = row-major [rows][cols/64] (file),
-                           // 1 = [ceil(rows/4)][cols/64][4] (4 rows per 8-byte load)
     RopeKV rope;           // kEpiRopeKV: interleaved RoPE of q/k rows, fp16 K/V append
     // In-launch rank-k projection (segments with k > 0 and tmp_k == null):
     // block b < sum(k) computes one tmp_k value and publishes it as one 64-bit

@@ -1762,7 +1762,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
         // another
         using KW = const __attribute__((address_space(4))) uint32_t;
         KW* kw = reinterpret_cast<KW*>(kargs);
-        static_assert(sizeof(HexArgs) <= 10 * 64, "argument lines touched below");
+        static_assert(sizeof(HexArgs) > 8 * 64 && sizeof(HexArgs) <= 9 * 64, "argument lines touched below");
         uint32_t t0 = kw[0], t1 = kw[16], t2 = kw[32], t3 = kw[48], t4 = kw[64];
         uint32_t t5 = kw[80], t6 = kw[96], t7 = kw[112], t8 = kw[128];
         uint32_t t9 = kw[(sizeof(HexArgs) - 4) / 4];
