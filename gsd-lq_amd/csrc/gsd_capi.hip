@@ -1032,7 +1032,7 @@ int issue_layer(gsdh_model* m, int l) {
 // projections, what issue_prefill computes: q, k and v in one launch, gate
 // and up in one, and each projection's column splits, descale, kink, rank-k,
 // residual and SwiGLU terms taken in by the pass that prepares the next
-// input.  9 launches per layer instead of 19.  The last layer forms what its
+// input.  10 launches per layer instead of 19.  The last layer forms what its
 // readers need: K and V of every token and, of the last token of the prompt
 // (`last`), the layer itself, by the decode step's launches; x is then the
 // last token's.  (The other tokens' attention, o and FFN of that layer have

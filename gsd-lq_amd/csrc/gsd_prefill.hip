@@ -75,18 +75,21 @@ __device__ __forceinline__ float mm_finish(const MmSeg& w, const MmIn& in, int m
 //    rows read half the fragments but run two per SIMD: 44-48 % of the matrix
 //    cores' cycles at 512 tokens, with either order of the reads, with raised
 //    priorities, and with the memory's latency taken out.)  923-token prompt
-//    3770 -> 3635 us;
+//    3790 -> 3494 us, both on one card (others: 3584 to 3770);
 //  * 32 x 32 tiles: one wave per SIMD issues 1.9 PFLOP/s of them and 1.1 of
 //    16 x 16 tiles (fp16, measured alone), two waves 2.06 against 1.72;
 //  * a lane's half of a 32-row tile comes from lanes (l & 15) + 32 (l >> 5)
 //    and + 16 of the two 16-row tiles in memory, so neither the weights nor
 //    the operands change their layout: step s = 2 q + t of a block takes
 //    lane group 2 (l >> 5) + q and codes 4 t .. 4 t + 3;
-//  * the tokens' fragments of a 64-column stage go from L2 straight into LDS
-//    (three stages, two in flight ahead of the one that is read), with one
-//    barrier per stage.  Through registers one stage ahead the latency of
-//    those loads took a third of the time (high + low, 28672 x 4096, 512
-//    tokens: 289 us, of which 118 went with the fragment loads);
+//  * the tokens' fragments of a 64-column stage go from L2 straight into LDS,
+//    three stages in turn, issued two ahead of the one that is read, with one
+//    barrier per stage.  (The copies of the next chunk's codes and scales at a
+//    chunk's end wait for all loads in the built loop: the first stage of a
+//    chunk is issued two stages before that wait, the second one.)  Through
+//    registers one stage ahead the latency of those loads took a third of the
+//    time (high + low, 28672 x 4096, 512 tokens: 289 us, of which 118 went with
+//    the fragment loads);
 //  * 32 copies of the codebook (128 bytes per entry) instead of 64: the half
 //    waves of a 4-byte LDS read are served in turn, and 28 KB for 217 points
 //    leave room for two blocks per CU.
@@ -96,8 +99,8 @@ __device__ __forceinline__ float mm_finish(const MmSeg& w, const MmIn& in, int m
 // 64 -> 37 us, 6144 x 4096 (q, k and v) at 37 tokens 23 -> 17 us.
 //
 // Safety of the LDS stages.  Stage n goes to buffer n % 3 two stages ahead.
-// A wave waits until only the younger loads than its share of stage n are in
-// flight (vmcnt counts in issue order: the share of stage n + 1, NF loads,
+// A wave waits at least until only the younger loads than its share of stage n
+// are in flight (vmcnt counts in issue order: the share of stage n + 1, NF loads,
 // and in the second stage of a chunk the 3 code and scale loads issued
 // after it) and for its own LDS reads, then meets the others; after that
 // barrier all of stage n is in LDS and no wave reads stage n - 1, whose
